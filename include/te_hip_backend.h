@@ -421,9 +421,9 @@ TE_API te_status te_hip_sample_top_k_f32(const float *logits, size_t vocab, uint
  * replaces.  pre: 0 none, 1 RMSNorm (norm_w, epsilon, as te_rmsnorm_f32),
  * 2 SwiGLU (x is gate, x2 is up, as te_swiglu_f32).  W is a GGUF Q4_0 (2) or
  * Q8_0 (8) tensor [n][k] in device memory at a 2-byte aligned address,
- * k % 32 == 0.  The activations are rounded per 32-value block to 15 bits of
- * the block's largest magnitude (error <= 2^-14 of it per value); products
- * are exact int8 MFMA sums, accumulated per block in fp32.  `act` is device
+ * k % 32 == 0.  Each activation enters as the sum of two bf16 values (error <=
+ * 2^-18 of it), each weight code exactly; products are bf16 MFMA sums in fp32,
+ * scaled and accumulated per 32-value block in fp32.  `act` is device
  * scratch of te_hip_gemm_act_bytes(rows, k) bytes.  `partials` (may be NULL)
  * is device scratch of partial_bytes bytes: with it, an output grid too small
  * to fill the GPU splits K into up to partial_bytes / (rows * n * 4) parts,
@@ -520,8 +520,7 @@ TE_API te_status te_hip_decode_layer_f16(
  *   - workspace: te_hip_prefill_all_layers_workspace_bytes(batch, hidden, kv,
  *     ffn) bytes, 256-byte aligned.
  * The projections are the batched-prefill GEMM (te_hip_gemm_q_f32: each
- * activation row rounded per 32-value block to 15 bits of its largest
- * magnitude, exact int8 MFMA products); the attention is
+ * activation as two bf16 parts, fp32 MFMA sums); the attention is
  * te_hip_attention_prefill_step_vt_f16.  Asynchronous on `stream`.  Checks as
  * te_hip_decode_all_layers_f16; Q4_0 / Q8_0 layer weights at 2-byte aligned
  * addresses only (other types or alignments -> UNSUPPORTED, the reference's

@@ -4,139 +4,50 @@
 // (reference c/src/qwen.c:630-905), whose per-row meaning is te_model_matvec_f32
 // (ops.c:177-269) applied to every row.
 //
-// Activations (quant_act_kernel): each row, after an optional RMSNorm or
-// SwiGLU pre-op, is cut into 32-value blocks.  A block of largest magnitude
-// m = f * 2^E (f in [0.5, 1)) is scaled by 2^(14-E) and rounded to integers v,
-// |v| <= 2^14, stored as two balanced int8 digits v = 256*hi + lo
-// (lo in [-128, 127]) plus the block scale 2^(E-14).  Rounding moves each value
-// by at most 2^-14 of its block's largest magnitude.
+// Products (gemm_bf16_kernel): one 32-value block of a row against one GGUF
+// block of a weight row is two K = 16 steps of v_mfma_f32_32x32x16_bf16 for
+// each of two operand parts.  An activation x enters as hi + lo bf16 (hi =
+// RNE(x), lo = RNE(x - hi): |x - hi - lo| <= 2^-18 |x|, with the exponent
+// range of fp32), a weight code (Q4_0's n - 8, Q8_0's byte) as one bf16,
+// exactly.  The block's fp32 sum is scaled by the weight block's scale d and
+// accumulated in fp32, one FMA per product of the block.
 //
-// Products (gemm_q_kernel): one 32-value block of a row against one GGUF
-// block of a weight row is a K = 32 step of v_mfma_i32_32x32x32_i8 -- the
-// integer sum of hi * q, shifted by 8, then the lo * q sum accumulated onto it
-// by a second MFMA: exact, |C| <= 32 * 2^14 * 128 < 2^31.  Each block's integer
-// result is scaled by (activation scale * weight block scale) and accumulated
-// in fp32.  Weight codes enter the MFMA as int8: Q8_0 as stored, Q4_0 nibbles
-// n as n - 8 (the reference's (q - 8) * d, ops.c:15-21).
+// Why two bf16 parts and not integer digits: a block-scaled integer digit
+// form (two int8 MFMAs at twice the rate) needs a shift, a conversion and the
+// product of two block scales for every sum, four VALU instructions per
+// output and block against 64 cycles of MFMA; a bf16 pair carries its own
+// exponent, so one FMA is left against 128 cycles of MFMA.
 //
-// Layout: the digit planes are stored in 32 x 32 tiles ([M/32][K/32][32 rows]
-// [32 k] int8), so one wave's operand for one block is 1 KiB contiguous.
+// Range: activations are stored times 2^-13 (kActScale) and the weight scales
+// times 2^13, so that a block's sum (32 products with codes up to 128) of
+// values near FLT_MAX stays finite, as the row's true sum does.
 //
-// Tiles: a 256-thread workgroup computes a 64 x 64 block of Y as four 32 x 32
-// wave tiles; the K loop takes two blocks per step (two independent MFMA
-// chains) and stages the activation scales of the workgroup's 64 rows in
-// LDS, 8 blocks at a time.  Where the output tiles alone would not fill the GPU,
-// the K range is split over grid.z and a second kernel adds the partial sums
-// in a fixed order (deterministic).
+// Layout of the activation operand (act_off): units of one 32-row tile and one
+// 32-value block, [M/32][K/32], 4 KiB each: [hi, lo][K step 0, 1][K half
+// 0, 1][32 rows][8 values] bf16 -- the order the MFMA operand is held in, so a
+// wave loads one operand as 1 KiB contiguous.
 #include "te_hip_common.h"
 
-#include <float.h>
+#include <math.h>
 
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
+#include "te_act_split.h"
+
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kQ4_0 = 2, kQ8_0 = 8;
 constexpr int kActThreads = 256;
-constexpr int kChunkBlocks = 8;
 
 __device__ __forceinline__ float half_bits(uint32_t bits) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
 }
 
 enum ActPre { kActPlain = 0, kActRmsNorm = 1, kActSwiGLU = 2 };
-
-// One 32-value block of digits: lane j of a half wave holds value j (every
-// lane of the half takes part; only `store` lanes write).
-__device__ __forceinline__ void quant_block(float v, size_t row, int K, int b, int lane, int8_t *__restrict__ hi,
-                                            int8_t *__restrict__ lo, float *__restrict__ scales, bool store = true) {
-    float m = fabsf(v);
-    for (int off = 16; off > 0; off >>= 1) {
-        m = fmaxf(m, __shfl_xor(m, off, 32));
-    }
-    int q = 0;
-    float s;
-    if (!(m <= FLT_MAX)) {  // inf or NaN in the block: its products are NaN
-        s = __builtin_nanf("");
-    } else if (m == 0.0f) {
-        s = 0.0f;
-    } else {
-        int E;
-        (void)frexpf(m, &E);
-        const int e = min(14 - E, 126);  // blocks below 2^-112 round towards 0
-        q = (int)rintf(ldexpf(v, e));
-        s = ldexpf(1.0f, -e);
-    }
-    if (store) {
-        const int l8 = ((q + 128) & 255) - 128;
-        const size_t t = (((row >> 5) * (size_t)(K >> 5) + b) << 10) + ((row & 31) << 5) + lane;
-        hi[t] = (int8_t)((q - l8) >> 8);
-        lo[t] = (int8_t)l8;
-        if (lane == 0) {
-            scales[row * (size_t)(K / 32) + b] = s;
-        }
-    }
-}
-
-// One 32-value block of digits held as eight consecutive values by each of
-// four adjacent lanes (g = lane & 3 holds values 8g .. 8g + 7): the same
-// digits and scale as quant_block (the block maximum does not depend on the
-// order it is taken in), stored as 8-byte pieces where `vec`.
-__device__ __forceinline__ void quant_block8(const float (&v)[8], size_t row, int K, int b, int g,
-                                             int8_t *__restrict__ hi, int8_t *__restrict__ lo,
-                                             float *__restrict__ scales, bool vec) {
-    float m = fabsf(v[0]);
-#pragma unroll
-    for (int j = 1; j < 8; ++j) {
-        m = fmaxf(m, fabsf(v[j]));
-    }
-    // the quad's maximum by DPP moves (lanes xor 1, then xor 2)
-    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0xB1, 0xF, 0xF, false)));
-    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x4E, 0xF, 0xF, false)));
-    int q[8] = {};
-    float s;
-    if (!(m <= FLT_MAX)) {  // inf or NaN in the block: its products are NaN
-        s = __builtin_nanf("");
-    } else if (m == 0.0f) {
-        s = 0.0f;
-    } else {
-        int E;
-        (void)frexpf(m, &E);
-        const int e = min(14 - E, 126);  // blocks below 2^-112 round towards 0
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            q[j] = (int)rintf(ldexpf(v[j], e));
-        }
-        s = ldexpf(1.0f, -e);
-    }
-    uint32_t h[2] = {0, 0}, l[2] = {0, 0};
-    // q = 256 * hi + lo with lo in [-128, 127]: hi = (q + 128) >> 8, and lo's
-    // byte is q's low byte
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        h[j >> 2] |= (uint32_t)(((q[j] + 128) >> 8) & 255) << (8 * (j & 3));
-        l[j >> 2] |= (uint32_t)(q[j] & 255) << (8 * (j & 3));
-    }
-    const size_t t = (((row >> 5) * (size_t)(K >> 5) + b) << 10) + ((row & 31) << 5) + 8 * g;
-    if (vec) {
-        *reinterpret_cast<uint2 *>(hi + t) = make_uint2(h[0], h[1]);
-        *reinterpret_cast<uint2 *>(lo + t) = make_uint2(l[0], l[1]);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            hi[t + j] = (int8_t)(h[j >> 2] >> (8 * (j & 3)));
-            lo[t + j] = (int8_t)(l[j >> 2] >> (8 * (j & 3)));
-        }
-    }
-    if (g == 0) {
-        scales[row * (size_t)(K / 32) + b] = s;
-    }
-}
 
 // Eight consecutive floats: two 16-byte loads where `vec`.
 __device__ __forceinline__ void load8(const float *p, bool vec, float (&v)[8]) {
@@ -167,7 +78,7 @@ __device__ __forceinline__ void store8(float *p, bool vec, const float (&v)[8]) 
 // The fp64 sum of squares of a row whose thread t holds columns
 // 8t + 2048i .. +7 (i = 0, 1, ...): each thread adds its values in column
 // order, the wave's lanes are added by an xor butterfly and the workgroup's
-// four waves in wave order.  quant_act_kernel<kActRmsNorm> and
+// four waves in wave order.  split_act_kernel<kActRmsNorm> and
 // gemm_reduce_rms_kernel both sum this way, so their RMSNorm factors agree
 // bit for bit.  (te_rmsnorm_f32, ops.c:272-293, sums in fp64 in index order.)
 __device__ __forceinline__ double row_sum_squares(double ss) {
@@ -187,21 +98,18 @@ __device__ __forceinline__ double row_sum_squares(double ss) {
     return t;
 }
 
-// x' = pre(x), then digits and block scales.  Thread t of a workgroup holds
+// x' = pre(x) as the GEMM's hi / lo operand.  Thread t of a workgroup holds
 // eight consecutive values of block t / 4 of a pass of 64 blocks; without a
 // row-wide norm the gridDim.y workgroups of a row take every gridDim.y-th
 // pass, else one workgroup takes the row (the norm's sum first, then the
-// digits from a second read of the row).
-// planes: hi and lo, int8 in 32 x 32 tiles [M/32][K/32][32][32]; scales [M][K/32] fp32.
-// `vec`: every pointer 16-byte aligned (16-byte loads, 8-byte digit stores).
+// operand from a second read of the row).  `vec`: the inputs are 16-byte
+// aligned.
 constexpr int kActPass = kActThreads * 8;
 template <int PRE>
-__global__ __launch_bounds__(kActThreads) void quant_act_kernel(const float *__restrict__ x,
+__global__ __launch_bounds__(kActThreads) void split_act_kernel(const float *__restrict__ x,
                                                                 const float *__restrict__ x2,
                                                                 const float *__restrict__ norm_w, float eps,
-                                                                int K, int8_t *__restrict__ hi,
-                                                                int8_t *__restrict__ lo,
-                                                                float *__restrict__ scales, bool vec) {
+                                                                int K, unsigned char *__restrict__ act, bool vec) {
     const size_t row = blockIdx.x;
     const float *xr = x + row * (size_t)K;
     const int c0 = 8 * (int)threadIdx.x;
@@ -235,151 +143,14 @@ __global__ __launch_bounds__(kActThreads) void quant_act_kernel(const float *__r
                 v[j] = v[j] / (1.0f + expf(-v[j])) * w2[j];  // te_swiglu_f32 (ops.c:397-405)
             }
         }
-        quant_block8(v, row, K, c >> 5, threadIdx.x & 3, hi, lo, scales, vec);
+        split_store8(v, row, K >> 5, c, act);
     }
 }
 
-// 16 weight codes of one GGUF block as int8: for Q4_0 the low (k < 16) or
-// high (k >= 16) nibbles of the 16 code bytes, n - 8; for Q8_0 the bytes
-// 16 * half .. +15.  `blk` is 2-byte aligned.
-template <uint32_t TYPE>
-__device__ __forceinline__ v4i weight_codes(const unsigned char *blk, int half, float &d) {
-    const uint16_t *h = reinterpret_cast<const uint16_t *>(blk);
-    d = half_bits(h[0]);
-    uint32_t w[4];
-    const int base = TYPE == kQ4_0 ? 1 : 1 + 8 * half;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        w[k] = (uint32_t)h[base + 2 * k] | (uint32_t)h[base + 2 * k + 1] << 16;
-    }
-    v4i out;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (TYPE == kQ4_0) {
-            // n ^ 8 is n - 8 as a 4-bit two's complement value; sign-extend per byte
-            const uint32_t x = ((half ? w[k] >> 4 : w[k]) & 0x0f0f0f0fu) ^ 0x08080808u;
-            out[k] = (int)(x | ((x & 0x08080808u) * 0x1eu));
-        } else {
-            out[k] = (int)w[k];
-        }
-    }
-    return out;
-}
-
-// grid (N/64, M/64, splits): split z covers blocks [z * per, (z + 1) * per).
-// With one split the result (+ resid) goes to `out`; otherwise the split's
-// partial sums go to part[z][M][N].
-template <uint32_t TYPE, bool RESID>
-__global__ __launch_bounds__(256) void gemm_q_kernel(const unsigned char *__restrict__ w, size_t row_bytes,
-                                                     const int8_t *__restrict__ hi, const int8_t *__restrict__ lo,
-                                                     const float *__restrict__ scales, int M, int N, int K, int per,
-                                                     float *out, const float *resid, float *part) {
-    constexpr int kBlockBytes = TYPE == kQ4_0 ? 18 : 34;
-    __shared__ __align__(16) float s_lds[kChunkBlocks][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int lr = lane & 31, kh = lane >> 5;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m_wg = blockIdx.y * 64;
-    const int m0 = m_wg + wm * 32, n0 = blockIdx.x * 64 + wn * 32;
-    const int b_col = min(n0 + lr, N - 1);
-    const int nb = K / 32;
-    const int kb0 = blockIdx.z * per, kb1 = min(nb, kb0 + per);
-    // rows of a partial 32-row tile read padding; their results are not stored
-    const size_t a_tile = (size_t)(min(m0, (M - 1) & ~31) >> 5) * nb;
-    const int a_lane = lr * 32 + kh * 16;
-    const unsigned char *b_row = w + (size_t)b_col * row_bytes;
-    float acc[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        acc[r] = 0.0f;
-    }
-    auto load = [&](int b, v4i &ah, v4i &al, v4i &bq, float &d) {
-        const size_t o = ((a_tile + b) << 10) + a_lane;
-        ah = *reinterpret_cast<const v4i *>(hi + o);
-        al = *reinterpret_cast<const v4i *>(lo + o);
-        bq = weight_codes<TYPE>(b_row + (size_t)b * kBlockBytes, kh, d);
-    };
-    // two blocks per step: two independent MFMA chains in flight
-    auto step = [&](int bb, const v4i &ah, const v4i &al, const v4i &bq, float d, v16i &c) {
-        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, bq, v16i{}, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            c[r] <<= 8;
-        }
-        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, bq, c, 0, 0, 0);
-        (void)bb;
-        (void)d;
-    };
-    auto scale_add = [&](int bb, const v16i &c, float d) {
-        // lane holds column lr of rows 8 * (r / 4) + 4 * kh + r % 4
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const float4 s4 = *reinterpret_cast<const float4 *>(&s_lds[bb][wm * 32 + 8 * g + 4 * kh]);
-            acc[4 * g + 0] = fmaf((float)c[4 * g + 0], s4.x * d, acc[4 * g + 0]);
-            acc[4 * g + 1] = fmaf((float)c[4 * g + 1], s4.y * d, acc[4 * g + 1]);
-            acc[4 * g + 2] = fmaf((float)c[4 * g + 2], s4.z * d, acc[4 * g + 2]);
-            acc[4 * g + 3] = fmaf((float)c[4 * g + 3], s4.w * d, acc[4 * g + 3]);
-        }
-    };
-    for (int b = kb0; b < kb1; b += 2) {
-        const int bb = (b - kb0) & (kChunkBlocks - 1);
-        if (bb == 0) {
-            __syncthreads();
-            for (int t = threadIdx.x; t < kChunkBlocks * 64; t += 256) {
-                const int rr = t & 63, cb = b + (t >> 6);
-                const int row = min(m_wg + rr, M - 1);
-                s_lds[t >> 6][rr] = cb < kb1 ? scales[(size_t)row * nb + cb] : 0.0f;
-            }
-            __syncthreads();
-        }
-        v4i ah0, al0, bq0, ah1, al1, bq1;
-        float d0, d1;
-        load(b, ah0, al0, bq0, d0);
-        const bool two = b + 1 < kb1;
-        if (two) {
-            load(b + 1, ah1, al1, bq1, d1);
-        }
-        v16i c0, c1;
-        step(bb, ah0, al0, bq0, d0, c0);
-        if (two) {
-            step(bb + 1, ah1, al1, bq1, d1, c1);
-        }
-        scale_add(bb, c0, d0);
-        if (two) {
-            scale_add(bb + 1, c1, d1);
-        }
-    }
-    const int col = n0 + lr;
-    if (col < N) {
-        float *dst = gridDim.z > 1 ? part + (size_t)blockIdx.z * M * N : out;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = m0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            if (row < M) {
-                const size_t o = (size_t)row * N + col;
-                dst[o] = RESID && gridDim.z == 1 ? resid[o] + acc[r] : acc[r];
-            }
-        }
-    }
-}
-
-// The same products with the weights staged through LDS: each K step takes a
-// chunk of kWChunk GGUF blocks of the workgroup's 64 weight rows, read as
-// 16-byte coalesced loads (a row's chunk is contiguous: 144 B for Q4_0, 272 B
-// for Q8_0, 16-byte aligned when the tensor and its row length are), one
-// chunk ahead of its use and double-buffered in LDS with a row pitch of an odd
-// dword count, so the wave's 32 rows read a block without bank conflicts.  A
-// lane's block (fp16 scale + codes) is a 5-dword LDS window whose byte
-// alignment is the same for every lane (the block index's parity), unpacked by
-// byte alignment and nibble masks.  Activation digits are prefetched one
-// block ahead.  Needs row_bytes % 16 == 0 and a 16-byte aligned tensor;
-// split boundaries fall on whole chunks.
-constexpr int kWChunk = 8;
-
-// Weight matrices of one launch (same K and type), whose 64-column tiles are
-// numbered one after another along grid.x: segment i holds tiles
-// tile_end[i-1] .. tile_end[i]-1.  Split-K partial sums are laid out
-// [split][segment][M][n] (n_off: columns before segment i).
+// Weight matrices of one launch (same K and type), whose column tiles are
+// numbered one after another: segment i holds tiles tile_end[i-1] ..
+// tile_end[i]-1.  Split-K partial sums are laid out [split][segment][M][n]
+// (n_off: columns before segment i).
 constexpr int kMaxGemmSegs = 3;
 struct GemmSegsArg {
     const unsigned char *w[kMaxGemmSegs];
@@ -391,258 +162,356 @@ struct GemmSegsArg {
     int nseg;
 };
 
-// GLU form's output: the SwiGLU of the paired gate / up products as the next
-// GEMM's activation digits (quant_act_kernel's planes and scales, K = n).
-struct GluDigits {
-    int8_t *hi;
-    int8_t *lo;
-    float *scales;
-};
+// Eight weight codes (int8 in two dwords) as bf16, exactly: int8 -> fp32, whose
+// upper half is the bf16.
+__device__ __forceinline__ uint4 codes_bf16(uint32_t c0, uint32_t c1) {
+    uint32_t f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int8_t q = (int8_t)((j < 4 ? c0 : c1) >> (8 * (j & 3)));
+        f[j] = __float_as_uint((float)(int)q);
+    }
+    uint4 r;
+    r.x = __builtin_amdgcn_perm(f[1], f[0], 0x07060302u);
+    r.y = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
+    r.z = __builtin_amdgcn_perm(f[5], f[4], 0x07060302u);
+    r.w = __builtin_amdgcn_perm(f[7], f[6], 0x07060302u);
+    return r;
+}
 
-// GLU = true: sg.w[0] / sg.w[1] are the gate / up matrices (n rows each) and
-// a workgroup's 64 weight rows pair the same 32 rows of both (wave wn = 0 the
-// gate products, wn = 1 the up products of the same 32 columns); the epilogue
-// forms silu(gate) * up with te_swiglu_f32's operations and writes its digits
-// (one 32-value block per row and workgroup), exactly as quant_act_kernel
-// would from the two products.  One K split.
-template <uint32_t TYPE, bool RESID, bool GLU>
-__global__ __launch_bounds__(256) void gemm_q2_kernel(GemmSegsArg sg, size_t row_bytes,
-                                                      const int8_t *__restrict__ hi, const int8_t *__restrict__ lo,
-                                                      const float *__restrict__ scales, int M, int K, int per,
-                                                      float *part, GluDigits glu) {
-    // this workgroup's segment (uniform)
+// Four nibbles (one per byte, 0..15) minus 8 as int8: (n + 0x78) ^ 0x80, no carries.
+__device__ __forceinline__ uint32_t nibbles_i8(uint32_t n) { return (n + 0x78787878u) ^ 0x80808080u; }
+
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// grid.x: (weight tile, split, row tile) units, see the index map below; 256 G
+// threads = G groups of 4 waves over BM = 32 * WM rows x 128 weight rows; a
+// wave's tile is 32 rows x (32 * WM) columns (WM = 4: a group's waves are
+// stacked over the rows and share the weight tile; WM = 2: two by two).  Two
+// groups take alternate chunks of K and add their sums through LDS at the end:
+// two waves per SIMD from one workgroup per CU, with half the split-K partial
+// sums of two one-group workgroups (the choice: gemm_plan).
+//
+// K runs in steps of G chunks of kCh blocks, one chunk per group.  Thread (n, p)
+// of the workgroup holds blocks 2p and 2p + 1 of weight row n of the next step
+// (36 / 68 bytes) in registers and converts them, a piece per step of the
+// second half, into the LDS buffer the group of p / 2 reads next
+// (double-buffered, one barrier per step).  LDS holds the converted operand in
+// MFMA order, [block][K step][32-row tile][K half][row] in 16-byte pieces (a
+// wave reads 1 KiB contiguous; the row's slot is xor 2p, so the 2 G
+// threads of a row store to different banks), and the scales d.  The activation
+// operand goes from global memory to registers, kCh - 1 blocks ahead.
+//
+// What bounds it: MFMA, VALU and the board's power together.  A loop of these
+// MFMAs alone on random operands runs at 1.75 PFLOP/s (the clock falls to 1.8
+// GHz); with the FMAs and LDS reads of a step 1.45, with the conversion 1.3.
+// Gate and up of 512 rows at 3B (2 x 11008 x 2048 Q4_0, 92 GFLOP of MFMA) take
+// 105 us, Q8_0 113 us, against 146 and 171 us with the block-scaled int8 digits
+// this replaced; converting the weights costs 15 us of it, their loads 5.
+//
+// GLU: sg.w[0] / sg.w[1] are the gate / up matrices (n rows each); the tile's
+// 128 weight rows are 32 gate, 32 up, 32 gate, 32 up, so a lane holds both
+// products of an output; the epilogue writes silu(gate) * up (te_swiglu_f32's
+// operations) as the next GEMM's operand.  One K split.
+//
+// W4: rows are 4-byte aligned and hold an even number of blocks; else the
+// blocks are read as 16-bit words.
+constexpr int kCh = 4;
+constexpr int kBN = 128;
+template <uint32_t TYPE, int WM, int G, bool GLU, bool W4>
+__global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void gemm_bf16_kernel(GemmSegsArg sg, size_t row_bytes,
+                                                           const unsigned char *__restrict__ act, int M, int K, int per,
+                                                           int m_tiles, int units, int n_tiles, float *part,
+                                                           unsigned char *glu_out) {
+    constexpr int BB = TYPE == kQ4_0 ? 18 : 34;  // bytes per GGUF block
+    constexpr int DW = 2 * BB / 4;               // dwords of a pair of blocks
+    constexpr int NT = WM;                       // 32-column tiles per wave
+    __shared__ __align__(16) uint4 wb_lds[G][2][kCh][2][2 * kBN];
+    __shared__ float sd_lds[G][2][kCh][kBN];
+    // Workgroups go to the XCDs round-robin; the row tiles of one (weight
+    // tile, split) unit stay on one XCD, whose L2 then reads its weights once.
+    const int xcd = (int)blockIdx.x & 7, slot_id = (int)blockIdx.x >> 3;
+    const int unit = slot_id / m_tiles * 8 + xcd;
+    const int m_t = slot_id % m_tiles;
+    if (unit >= units) {
+        return;
+    }
+    const int z = unit / n_tiles, tile = unit % n_tiles;
     int seg = 0;
 #pragma unroll
     for (int i = 1; i < kMaxGemmSegs; ++i) {
-        seg += (i < sg.nseg && (int)blockIdx.x >= sg.tile_end[i - 1]) ? 1 : 0;
+        seg += (i < sg.nseg && tile >= sg.tile_end[i - 1]) ? 1 : 0;
     }
-    const unsigned char *__restrict__ w = sg.w[seg];
     const int N = sg.n[seg];
-    float *out = sg.out[seg];
-    const float *resid = sg.resid[seg];
-    const int n_tile = (int)blockIdx.x - (seg > 0 ? sg.tile_end[seg - 1] : 0);
-    const uintptr_t up_delta = GLU ? (uintptr_t)sg.w[1] - (uintptr_t)sg.w[0] : 0;  // modulo 2^64
-    constexpr int BB = TYPE == kQ4_0 ? 18 : 34;     // bytes per GGUF block
-    constexpr int CB = kWChunk * BB;                // bytes of one row's chunk
-    constexpr int PITCH = CB + 4;                   // LDS row pitch (CB is a multiple of 16)
-    constexpr int RC = CB / 16;                     // 16-byte pieces per row chunk
-    constexpr int PIECES = 64 * RC;
-    constexpr int PPT = (PIECES + 255) / 256;       // pieces per thread
-    static_assert(CB % 16 == 0 && (PITCH / 4) % 2 == 1, "chunk layout");
-    __shared__ __align__(16) unsigned char w_lds[2][64 * PITCH];
-    __shared__ __align__(16) float s_lds[2][kWChunk][64];
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+    const int n_wg = (tile - (seg > 0 ? sg.tile_end[seg - 1] : 0)) * (GLU ? kBN / 2 : kBN);
+    const int tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
+    const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
     const int lr = lane & 31, kh = lane >> 5;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m_wg = blockIdx.y * 64, n_wg = n_tile * (GLU ? 32 : 64);
-    const int m0 = m_wg + wm * 32, n0 = GLU ? n_wg : n_wg + wn * 32;
+    const int wm = wave % WM, wn = wave / WM;
+    const int m0 = (m_t * WM + wm) * 32;
+    const bool active = m0 < M;
     const int nb = K / 32;
-    const int kb0 = blockIdx.z * per, kb1 = min(nb, kb0 + per);
-    const size_t a_tile = (size_t)(min(m0, (M - 1) & ~31) >> 5) * nb;
-    const int a_lane = lr * 32 + kh * 16;
-    const int n_chunks = (kb1 - kb0 + kWChunk - 1) / kWChunk;
+    const int kb0 = z * per, kb1 = min(nb, kb0 + per);
+    // chunks of each group: chunk c is blocks kb0 + (G c + group) kCh ..; past
+    // kb1 the weights are zeros
+    const int n_chunks = (kb1 - kb0 + G * kCh - 1) / (G * kCh);
+    auto &wb = wb_lds[group];
+    auto &sd = sd_lds[group];
 
-    // chunk c's pieces and activation scales: global -> registers (a chunk
-    // ahead), then registers -> LDS buffer. Q8_0 stages its 5 pieces per
-    // thread in two halves (the first stored and the second loaded at the
-    // chunk's midpoint): only 3 pieces are held in registers, which keeps the
-    // kernel at <= 128 VGPRs (4 waves per SIMD instead of 3). Q4_0 (3 pieces)
-    // stages the chunk at once: halves measured slower there.
-    constexpr int SPT = kWChunk * 64 / 256;  // scales per thread
-    constexpr bool HALVES = TYPE == kQ8_0;
-    constexpr int PA = HALVES ? (PPT + 1) / 2 : PPT;  // pieces of the first half
-    using P0 = std::integral_constant<int, 0>;
-    using PMid = std::integral_constant<int, PA>;
-    using PEnd = std::integral_constant<int, PPT>;
-    using PLast = std::integral_constant<int, HALVES ? PA : 0>;  // first piece stored at the chunk's end
-    uint4 wreg[PA];
-    float sreg[SPT];
-    auto load_scales = [&](int c) {
+    // ---- weights: global -> registers -> converted in LDS
+    // (the 2 G threads of a row read consecutive blocks, the groups' next
+    // chunks; sp: the pair of blocks, of group sp / 2)
+    const int sn = (int)threadIdx.x / (2 * G), sp = (int)threadIdx.x % (2 * G);
+    auto &wb_st = wb_lds[sp >> 1];
+    auto &sd_st = sd_lds[sp >> 1];
+    const unsigned char *wrow;
+    {
+        const int i = sn >> 5;
+        const int row = min(GLU ? n_wg + (i >> 1) * 32 + (sn & 31) : n_wg + sn, N - 1);
+        wrow = (GLU ? sg.w[i & 1] : sg.w[seg]) + (size_t)row * row_bytes;
+    }
+    uint32_t wreg[DW];
+    // load i of chunk c's pair (kLoads in all): 16 bytes, the last one dword.
+    // Blocks past the split's end are read from its last ones (no branch
+    // around the loads) and get the scale 0.
+    constexpr int kLoads = (DW + 3) / 4;
+    auto load_w = [&](int c, int i) {
+        const int b = kb0 + G * c * kCh + 2 * sp;
+        if (W4) {
+            const unsigned char *p = wrow + (size_t)min(b, kb1 - 2) * BB;
+            if (4 * i + 4 <= DW) {
+                const u32x4_a4 v = *reinterpret_cast<const u32x4_a4 *>(p + 16 * i);
+                wreg[4 * i] = v[0], wreg[4 * i + 1] = v[1], wreg[4 * i + 2] = v[2], wreg[4 * i + 3] = v[3];
+            } else {
+                wreg[DW - 1] = *reinterpret_cast<const uint32_t *>(p + 4 * (DW - 1));
+            }
+        } else {
+            const uint16_t *h0 = reinterpret_cast<const uint16_t *>(wrow + (size_t)min(b, kb1 - 1) * BB);
+            const uint16_t *h1 = reinterpret_cast<const uint16_t *>(wrow + (size_t)min(b + 1, kb1 - 1) * BB);
+            uint32_t half[8] = {};
 #pragma unroll
-        for (int i = 0; i < SPT; ++i) {
-            const int t = tid + 256 * i;
-            const int rr = t & 63, cb = kb0 + c * kWChunk + (t >> 6);
-            const int row = min(m_wg + rr, M - 1);
-            sreg[i] = cb < kb1 ? scales[(size_t)row * nb + cb] : 0.0f;
-        }
-    };
-    // pieces I0 .. I1 - 1 of chunk c into wreg[0 ..]
-    auto load_pieces = [&](int c, auto i0, auto i1) {
-        constexpr int I0 = decltype(i0)::value, I1 = decltype(i1)::value;
-        const size_t cbyte = (size_t)(kb0 + c * kWChunk) * BB;
+            for (int k = 0; k < 8; ++k) {
+                const int e = 8 * i + k;  // 16-bit word of the pair
+                if (e < BB) {
+                    half[k] = e < BB / 2 ? h0[e] : h1[e - BB / 2];
+                }
+            }
 #pragma unroll
-        for (int i = I0; i < I1; ++i) {
-            const int item = tid + 256 * i;
-            const int r = item / RC, j = item % RC;
-            const size_t off = cbyte + 16 * (size_t)j;
-            wreg[i - I0] = make_uint4(0u, 0u, 0u, 0u);
-            if (item < PIECES && off < row_bytes) {  // a piece is wholly in its row or wholly past it
-                // GLU: rows 0..31 of the tile from the gate matrix, 32..63 from
-                // up (a byte offset from gate: a per-piece pointer select
-                // costs registers that lower occupancy)
-                const int row = min(n_wg + (GLU ? (r & 31) : r), N - 1);
-                const uintptr_t base = (uintptr_t)w + (GLU ? (uintptr_t)(r >> 5) * up_delta : 0);
-                wreg[i - I0] = *reinterpret_cast<const uint4 *>(base + (size_t)row * row_bytes + off);
+            for (int k = 0; k < 4; ++k) {
+                if (4 * i + k < DW) {
+                    wreg[4 * i + k] = half[2 * k] | half[2 * k + 1] << 16;
+                }
             }
         }
     };
-    auto store_pieces = [&](int buf, auto i0, auto i1) {
-        constexpr int I0 = decltype(i0)::value, I1 = decltype(i1)::value;
-#pragma unroll
-        for (int i = I0; i < I1; ++i) {
-            const int item = tid + 256 * i;
-            if (item < PIECES) {
-                uint32_t *dst = reinterpret_cast<uint32_t *>(&w_lds[buf][(item / RC) * PITCH + 16 * (item % RC)]);
-                dst[0] = wreg[i - I0].x;
-                dst[1] = wreg[i - I0].y;
-                dst[2] = wreg[i - I0].z;
-                dst[3] = wreg[i - I0].w;
-            }
+    // piece q of the thread's pair of blocks: its block q / 4, K step (q / 2) % 2,
+    // K half q % 2; piece 0 of a block also stores its scale
+    constexpr int kPieces = 8;
+    auto store_w = [&](int c, int buf, int q) {
+        const int i = q >> 2, s = (q >> 1) & 1, h = q & 1;
+        const int blk = 2 * (sp & 1) + i;
+        if ((q & 3) == 0) {
+            const float d = half_bits(i == 0 ? wreg[0] & 0xffffu : wreg[BB / 4] >> 16) * kActUnscale;
+            sd_st[buf][blk][sn] = kb0 + G * c * kCh + 2 * sp + i < kb1 ? d : 0.0f;
         }
-    };
-    auto store_scales = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < SPT; ++i) {
-            const int t = tid + 256 * i;
-            s_lds[buf][t >> 6][t & 63] = sreg[i];
+        auto code = [&](int k) {  // dword k of the block's codes
+            return i == 0 ? __builtin_amdgcn_alignbyte(wreg[k + 1], wreg[k], 2) : wreg[BB / 4 + 1 + k];
+        };
+        uint4 v;
+        if (TYPE == kQ4_0) {
+            v = codes_bf16(nibbles_i8((code(2 * h) >> (4 * s)) & 0x0f0f0f0fu),
+                           nibbles_i8((code(2 * h + 1) >> (4 * s)) & 0x0f0f0f0fu));
+        } else {
+            v = codes_bf16(code(4 * s + 2 * h), code(4 * s + 2 * h + 1));
         }
+        wb_st[buf][blk][s][64 * (sn >> 5) + 32 * h + ((sn & 31) ^ (2 * sp))] = v;
     };
-    // activation digits of block b, one block ahead of use (two ahead took 8
-    // more VGPRs and measured 3-4 % slower)
-    v4i ah[2], al[2];
-    auto load_a = [&](int b, int slot) {
-        if (b < kb1) {
-            const size_t o = ((a_tile + b) << 10) + a_lane;
-            ah[slot] = *reinterpret_cast<const v4i *>(hi + o);
-            al[slot] = *reinterpret_cast<const v4i *>(lo + o);
-        }
+
+    // ---- activations: global -> registers, kCh - 1 blocks ahead
+    const unsigned char *a_base = act + (((size_t)(min(m0, (M - 1) & ~31) >> 5) * nb) << 12) + lane * 16;
+    uint4 areg[kCh][4];
+    auto load_a = [&](int b, int slot, int i) {
+        areg[slot][i] = *reinterpret_cast<const uint4 *>(a_base + ((size_t)min(b, kb1 - 1) << 12) + 1024 * i);
     };
-    float acc[16];
+
+    // A step is one 32 x 32 tile of one block: four MFMAs, under which the
+    // previous step's sums are scaled and added, the next step's weights are
+    // read from LDS and (second half of a chunk) a piece of the next chunk is
+    // converted.
+    constexpr int kSteps = kCh * NT;
+    v16f acc[NT], prev = {};
+    float prev_d = 0.0f;
+    bf16x8 bw[2][2];
+    float bd[2];
+    auto load_b = [&](int buf, int step) {
+        const int bb = step / NT, tile = wn * NT + step % NT, slot = 64 * tile + (lane ^ (4 * group + 2 * (bb >> 1)));
+        bw[step & 1][0] = __builtin_bit_cast(bf16x8, wb[buf][bb][0][slot]);
+        bw[step & 1][1] = __builtin_bit_cast(bf16x8, wb[buf][bb][1][slot]);
+        bd[step & 1] = sd[buf][bb][32 * tile + lr];
+    };
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        acc[r] = 0.0f;
+    for (int t = 0; t < NT; ++t) {
+        acc[t] = v16f{};
     }
     if (n_chunks > 0) {
-        load_scales(0);
-        load_pieces(0, P0{}, PMid{});
-        store_pieces(0, P0{}, PMid{});
-        load_pieces(0, PMid{}, PEnd{});
-        store_pieces(0, PMid{}, PEnd{});
-        store_scales(0);
-        load_a(kb0, 0);
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            load_w(0, i);
+        }
+#pragma unroll
+        for (int i = 0; i < 4 * (kCh - 1); ++i) {
+            load_a(kb0 + group * kCh + i / 4, i / 4, i % 4);
+        }
+#pragma unroll
+        for (int q = 0; q < kPieces; ++q) {
+            store_w(0, 0, q);
+        }
     }
     __syncthreads();
     for (int c = 0; c < n_chunks; ++c) {
         const int buf = c & 1;
-        if (c + 1 < n_chunks) {
-            load_scales(c + 1);
-            load_pieces(c + 1, P0{}, PMid{});
-        }
-        const unsigned char *wrow = &w_lds[buf][(wn * 32 + lr) * PITCH];
+        load_b(buf, 0);
 #pragma unroll
-        for (int bb = 0; bb < kWChunk; ++bb) {
-            const int b = kb0 + c * kWChunk + bb;
-            load_a(b + 1, (bb + 1) & 1);
-            if (HALVES && bb == kWChunk / 2 && c + 1 < n_chunks) {
-                // buffer buf ^ 1 was last read before the previous chunk's barrier
-                store_pieces(buf ^ 1, P0{}, PMid{});
-                load_pieces(c + 1, PMid{}, PEnd{});
+        for (int step = 0; step < kSteps; ++step) {
+            const int bb = step / NT, t = step % NT;
+            // One step's share of the global loads: a burst of them would hold
+            // the wave (and, in step with it, the others) at their issue.
+            // Activations are kCh - 1 blocks ahead: loads return in order, so
+            // waiting for activations issued after the weights (from HBM) waits
+            // for the weights too.  The last chunk loads and converts itself
+            // again, which nothing reads.
+#pragma unroll
+            for (int i = 0; i < 4 / NT; ++i) {
+                load_a(kb0 + (G * c + group) * kCh + (bb == 0 ? kCh - 1 : G * kCh + bb - 1), (bb + kCh - 1) % kCh,
+                       t * (4 / NT) + i);
             }
-            if (b < kb1) {
-                // the block's fp16 scale and 16 codes of this lane's k half: a
-                // 5-dword window starting at the block's dword (Q8_0: the half's)
-                const int blk = bb * BB;                                  // compile-time per bb
-                const int start = TYPE == kQ4_0 ? blk : blk + 16 * kh;   // the lane's codes are at start + 2
-                const uint32_t *win = reinterpret_cast<const uint32_t *>(wrow + (start & ~3));
-                uint32_t dw[5];
 #pragma unroll
-                for (int i = 0; i < 5; ++i) {
-                    dw[i] = win[i];
-                }
-                // fp16 scale: bytes blk, blk + 1 (the same dword as the window's
-                // first for Q4_0)
-                const uint32_t dwin =
-                    TYPE == kQ4_0 ? dw[0] : *reinterpret_cast<const uint32_t *>(wrow + (blk & ~3));
-                const float d = half_bits((blk & 2) ? dwin >> 16 : dwin & 0xffffu);
-                // codes: bytes start + 2 + 4k .. +3 for k = 0..3, at byte 2 or 4
-                // of the window (blk is 0 or 2 mod 4, as start is)
-                const int sh = (blk & 3) + 2;
-                uint32_t code[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    code[k] = sh == 4 ? dw[k + 1] : __builtin_amdgcn_alignbyte(dw[k + 1], dw[k], 2);
-                }
-                v4i bq;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (TYPE == kQ4_0) {
-                        // per byte n in 0..15: (n + 0x78) ^ 0x80 is n - 8 as int8
-                        // (no byte carries: n + 0x78 <= 0x87)
-                        const uint32_t n4 = (kh ? code[k] >> 4 : code[k]) & 0x0f0f0f0fu;
-                        bq[k] = (int)((n4 + 0x78787878u) ^ 0x80808080u);
-                    } else {
-                        bq[k] = (int)code[k];
-                    }
-                }
-                const int slot = bb & 1;
-                v16i cc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[slot], bq, v16i{}, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    cc[r] <<= 8;
-                }
-                cc = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[slot], bq, cc, 0, 0, 0);
-                // lane holds column lr of rows 8 * (r / 4) + 4 * kh + r % 4
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const float4 s4 = *reinterpret_cast<const float4 *>(&s_lds[buf][bb][wm * 32 + 8 * g + 4 * kh]);
-                    acc[4 * g + 0] = fmaf((float)cc[4 * g + 0], s4.x * d, acc[4 * g + 0]);
-                    acc[4 * g + 1] = fmaf((float)cc[4 * g + 1], s4.y * d, acc[4 * g + 1]);
-                    acc[4 * g + 2] = fmaf((float)cc[4 * g + 2], s4.z * d, acc[4 * g + 2]);
-                    acc[4 * g + 3] = fmaf((float)cc[4 * g + 3], s4.w * d, acc[4 * g + 3]);
+            for (int i = 0; i < kLoads; ++i) {
+                if (step == i * (kSteps / 2) / kLoads) {
+                    load_w(min(c + 1, n_chunks - 1), i);
                 }
             }
-        }
-        if (c + 1 < n_chunks) {
-            store_pieces(buf ^ 1, PLast{}, PEnd{});
-            store_scales(buf ^ 1);
+            if (step + 1 < kSteps) {
+                load_b(buf, step + 1);
+            }
+            // the loads are issued here, not sunk towards their use
+            __builtin_amdgcn_sched_barrier(0);
+            const bf16x8 b0 = bw[step & 1][0], b1 = bw[step & 1][1];
+            v16f s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, areg[bb][0]), b0, v16f{},
+                                                             0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, areg[bb][1]), b1, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, areg[bb][2]), b0, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, areg[bb][3]), b1, s, 0, 0, 0);
+            const int tp = (t + NT - 1) % NT;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[tp][r] = fmaf(prev[r], prev_d, acc[tp][r]);
+            }
+            // pieces over the second half of the chunk's steps
+            constexpr int kPer = kPieces / (kSteps / 2);
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                if (step >= kSteps / 2) {
+                    store_w(min(c + 1, n_chunks - 1), buf ^ 1, (step - kSteps / 2) * kPer + i);
+                }
+            }
+            prev = s;
+            prev_d = bd[step & 1];
+            __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
     }
-    const int col = n0 + lr;
-    if constexpr (GLU) {
-        // up products -> LDS (the weight stages are free after the last
-        // barrier); the gate wave forms h and its digits
-        float *xch = reinterpret_cast<float *>(&w_lds[0][0]);
-        static_assert(sizeof(w_lds) >= 2 * 16 * 64 * sizeof(float), "exchange fits the weight stages");
-        if (wn == 1) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                xch[(wm * 16 + r) * 64 + lane] = acc[r];
+    for (int r = 0; r < 16; ++r) {
+        acc[NT - 1][r] = fmaf(prev[r], prev_d, acc[NT - 1][r]);
+    }
+    // Each group finishes the tiles it owns: the other's sums of them come
+    // through LDS (group 0's first, then group 1's)
+    auto owns = [&](int g, int t) { return G == 1 || (NT == 4 ? t / 2 == g : GLU ? g == 0 : t == g); };
+    if constexpr (G == 2) {
+        float4 *xs = reinterpret_cast<float4 *>(&wb_lds[0][0][0][0][0]);
+        static_assert(sizeof(wb_lds) >= NT * 4 * 16 * 64 * sizeof(float), "the exchange fits the weight stages");
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if (!owns(group, t)) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    xs[((t * 4 + wave) * 4 + q) * 64 + lane] =
+                        make_float4(acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]);
+                }
             }
         }
         __syncthreads();
-        if (wn == 0) {
-            const int b = n_wg >> 5;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if (owns(group, t)) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 v = xs[((t * 4 + wave) * 4 + q) * 64 + lane];
+                    acc[t][4 * q] += v.x, acc[t][4 * q + 1] += v.y, acc[t][4 * q + 2] += v.z, acc[t][4 * q + 3] += v.w;
+                }
+            }
+        }
+    }
+    // lane holds column lr of rows 8 * (r / 4) + 4 * kh + r % 4 of each 32 x 32 tile
+    if constexpr (GLU) {
+        // silu(gate) * up, split and turned through LDS into the operand's
+        // order (rows of 32 + 1 dwords: hi | lo << 16)
+        uint32_t *xch = reinterpret_cast<uint32_t *>(&wb_lds[G - 1][0][0][0][0]) + (group * 4 + wave) * (32 * 33);
+        static_assert(sizeof(wb_lds[0]) >= NT * 4 * 16 * 64 * sizeof(float) && sizeof(wb_lds[0]) >= G * 4 * 32 * 33 * 4,
+                      "the exchange and the turned tiles each fit one group's weight stages");
+        const int nb_out = N / 32;
+#pragma unroll
+        for (int p = 0; p < NT / 2; ++p) {
+            const int b = n_wg / 32 + wn * (NT / 2) + p;
+            if (!owns(group, 2 * p) || !active || b >= nb_out) {
+                continue;
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int row = m0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-                const float g = acc[r];
-                const float u = xch[(wm * 16 + r) * 64 + lane];
+                const float g = acc[2 * p][r], u = acc[2 * p + 1][r];
                 const float v = g / (1.0f + expf(-g)) * u;  // te_swiglu_f32 (ops.c:397-405)
-                quant_block(v, (size_t)row, N, b, lr, glu.hi, glu.lo, glu.scales, row < M);
+                xch[(8 * (r >> 2) + 4 * kh + (r & 3)) * 33 + lr] = split_pack(v);
+            }
+            // only this wave's own slice: its writes before its reads
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            unsigned char *dst = glu_out + (((size_t)(m0 >> 5) * nb_out + b) << 12) + lane * 16;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint32_t e[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    e[j] = xch[lr * 33 + 16 * s + 8 * kh + j];
+                }
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    hi[j] = __builtin_amdgcn_perm(e[2 * j + 1], e[2 * j], 0x05040100u);
+                    lo[j] = __builtin_amdgcn_perm(e[2 * j + 1], e[2 * j], 0x07060302u);
+                }
+                *reinterpret_cast<uint4 *>(dst + 1024 * s) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                *reinterpret_cast<uint4 *>(dst + 2048 + 1024 * s) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
             }
         }
         return;
     }
-    if (col < N) {
-        float *dst = gridDim.z > 1 ? part + ((size_t)blockIdx.z * sg.n_off[sg.nseg] + sg.n_off[seg]) * M : out;
+    if (!active) {
+        return;
+    }
+    const bool one = units == n_tiles;  // one split
+    float *dst = one ? sg.out[seg] : part + ((size_t)z * sg.n_off[sg.nseg] + sg.n_off[seg]) * M;
+    const float *resid = one ? sg.resid[seg] : nullptr;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = m0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            if (row < M) {
-                const size_t o = (size_t)row * N + col;
-                dst[o] = RESID && gridDim.z == 1 ? resid[o] + acc[r] : acc[r];
+    for (int t = 0; t < NT; ++t) {
+        const int col = n_wg + 32 * (wn * NT + t) + lr;
+        if (owns(group, t) && col < N) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = m0 + 8 * (r >> 2) + 4 * kh + (r & 3);
+                if (row < M) {
+                    const size_t o = (size_t)row * N + col;
+                    dst[o] = resid != nullptr ? resid[o] + acc[t][r] : acc[t][r];
+                }
             }
         }
     }
@@ -727,21 +596,19 @@ __global__ __launch_bounds__(256) void gemm_reduce_segs_kernel(const float *__re
 }
 
 // gemm_reduce_kernel's sums for one row (resid + the splits' partial sums in
-// split order -> out), then that row's RMSNorm digits into hi / lo / scales,
-// exactly as quant_act_kernel<kActRmsNorm> computes them from out: thread t
-// holds columns 8t .. 8t + 7, summed into the fp64 sum of squares in
-// row_sum_squares's order, and quantizes them as quant_act_kernel's thread t
-// does.  One workgroup per row, N <= kActPass, N % 32 == 0,
+// split order -> out), then that row's RMSNorm operand into act, exactly as
+// split_act_kernel<kActRmsNorm> computes it from out: thread t holds columns
+// 8t .. 8t + 7, summed into the fp64 sum of squares in row_sum_squares's order,
+// and splits them as split_act_kernel's thread t does.  One workgroup per row, N <= kActPass, N % 32 == 0,
 // splits <= kRmsSplits.  Every load, the norm weights' included, is issued
 // before the first store (out may be resid), so all of a thread's loads are
 // in flight together.
-constexpr int kRmsSplits = 8;
+constexpr int kRmsSplits = 16;  // also the most splits of a launch
 __global__ __launch_bounds__(kActThreads) void gemm_reduce_rms_kernel(const float *__restrict__ part, int splits,
                                                                       size_t count, const float *resid, float *out,
                                                                       int N, const float *__restrict__ norm_w,
-                                                                      float eps, int8_t *__restrict__ hi,
-                                                                      int8_t *__restrict__ lo,
-                                                                      float *__restrict__ scales, bool vec) {
+                                                                      float eps, unsigned char *__restrict__ act,
+                                                                      bool vec) {
     const size_t row = blockIdx.x;
     const int c = 8 * (int)threadIdx.x;
     const bool mine = c < N;
@@ -782,7 +649,7 @@ __global__ __launch_bounds__(kActThreads) void gemm_reduce_rms_kernel(const floa
         for (int j = 0; j < 8; ++j) {
             xv[j] = xv[j] * rms * wv[j];
         }
-        quant_block8(xv, row, N, c >> 5, threadIdx.x & 3, hi, lo, scales, vec);
+        split_store8(xv, row, N >> 5, c, act);
     }
 }
 
@@ -813,42 +680,124 @@ static bool aligned16(const void *p) {
     return ((uintptr_t)p & 15u) == 0;
 }
 
-// digit planes padded to whole 32-row tiles
-static size_t plane_bytes(size_t rows, size_t cols) {
-    return (rows + 31) / 32 * 32 * cols;
-}
+// 32-row tiles, hi and lo; 16 bytes so that any pointer has an aligned base
+size_t act_buffer_bytes(size_t rows, size_t cols) { return (rows + 31) / 32 * 32 * cols * 4 + 16; }
 
-size_t act_plane_bytes(size_t rows, size_t cols) {
-    return plane_bytes(rows, cols);
-}
-
-size_t act_buffer_bytes(size_t rows, size_t cols) {
-    return 2 * plane_bytes(rows, cols) + rows * (cols / 32) * sizeof(float);
-}
-
-te_status launch_quant_act(int pre, const float *x, const float *x2, const float *norm_w, float eps, size_t rows,
+te_status launch_split_act(int pre, const float *x, const float *x2, const float *norm_w, float eps, size_t rows,
                            size_t cols, void *act, hipStream_t stream) {
     if (rows == 0 || cols == 0 || cols % 32 != 0 || rows > 0x7fffffffu || cols > (1u << 24)) {
         return TE_STATUS_UNSUPPORTED;
     }
-    const size_t planes = plane_bytes(rows, cols);
-    int8_t *hi = static_cast<int8_t *>(act);
-    int8_t *lo = hi + planes;
-    float *scales = reinterpret_cast<float *>(lo + planes);
-    const bool vec = aligned16(x) && aligned16(act) && (pre != kActSwiGLU || aligned16(x2)) &&
-                     (pre != kActRmsNorm || aligned16(norm_w));
+    unsigned char *a = act_base(act);
+    const bool vec = aligned16(x) && (pre != kActSwiGLU || aligned16(x2)) && (pre != kActRmsNorm || aligned16(norm_w));
     // without a row-wide norm, the row's passes of kActPass values are spread over workgroups
     const dim3 grid((unsigned)rows, pre == kActRmsNorm ? 1u : (unsigned)std::max<size_t>(1, cols / kActPass));
     if (pre == kActRmsNorm) {
-        quant_act_kernel<kActRmsNorm>
-            <<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, hi, lo, scales, vec);
+        split_act_kernel<kActRmsNorm><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, a, vec);
     } else if (pre == kActSwiGLU) {
-        quant_act_kernel<kActSwiGLU><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, hi, lo, scales, vec);
+        split_act_kernel<kActSwiGLU><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, a, vec);
     } else {
-        quant_act_kernel<kActPlain><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, hi, lo, scales, vec);
+        split_act_kernel<kActPlain><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, a, vec);
     }
     return launch_status();
 }
+
+// Rows per workgroup (32 * wm), groups per workgroup, K splits and their
+// length, from the estimated time of a launch.  A (weight tile, split) unit and
+// its row tiles stay on one XCD, so the rounds of one workgroup per CU are
+// counted per XCD (28 weight tiles x 3 splits x 3 row tiles: 252 workgroups,
+// but 33 on some XCDs, measured 145 us against 111 with 2 splits).
+//   One round: two groups per workgroup.  A pair of chunks takes 3.4 us at 128
+//   rows on 64 CUs and 4.9 on all 256 (the clock falls), 2.5 and 3.0 at 64.
+//   More: two one-group workgroups per CU, which fill each other's waits (512
+//   x 22016 x 2048 Q4_0 109.7 us against 120.2 in two-group workgroups, Q8_0
+//   118.3 against 129.7); a round's pair takes 4.2 and 2.8 us.
+// The partial sums are written and read back at 2.7 TB/s.
+struct GemmPlan {
+    int wm, groups;
+    size_t per, splits;  // blocks of K per split, a multiple of two chunks
+};
+static GemmPlan gemm_plan(size_t rows, size_t n, size_t n_tiles, size_t nb, size_t splits_max) {
+    const size_t pairs = (nb + 2 * kCh - 1) / (2 * kCh);
+    const double cus = (double)device_compute_units();
+    GemmPlan best = {};
+    double best_us = 0.0;
+    for (int wm = 2; wm <= 4; wm += 2) {
+        const size_t m_tiles = (rows + 32 * wm - 1) / (32 * wm);
+        for (size_t want = 1; want <= std::min<size_t>(splits_max, kRmsSplits); ++want) {
+            const size_t per = (pairs + want - 1) / want;
+            const size_t splits = (pairs + per - 1) / per;
+            const double per_xcd = (double)((n_tiles * splits + 7) / 8 * m_tiles);
+            const double rounds = ceil(per_xcd * 8.0 / cus);
+            const double busy = std::min(1.0, per_xcd * 8.0 / cus);
+            const double pair_us = rounds > 1.0 ? (wm == 4 ? 4.2 : 2.8) : wm == 4 ? 3.0 + 1.9 * busy : 2.1 + 0.9 * busy;
+            const double us = rounds * (pair_us * (double)per + 3.5) +
+                              (splits > 1 ? 2.0 + (double)(splits * rows * n) * 8.0 / 2.7e6 : 0.0);
+            if (best.wm == 0 || us < best_us) {
+                best_us = us;
+                best = {wm, rounds > 1.0 ? 1 : 2, per * 2 * kCh, splits};
+            }
+        }
+    }
+    return best;
+}
+
+// One gemm_bf16_kernel launch.
+static te_status launch_tiles(uint32_t ggml_type, bool glu, bool w4, const GemmSegsArg &sg, size_t row_bytes,
+                              const void *act, size_t rows, size_t k, const GemmPlan &plan, size_t n_tiles,
+                              float *part, void *glu_out, hipStream_t stream) {
+    const size_t wm = (size_t)plan.wm;
+    const size_t m_tiles = (rows + 32 * wm - 1) / (32 * wm);
+    const size_t units = n_tiles * plan.splits;
+    const size_t blocks = (units + 7) / 8 * 8 * m_tiles;
+    if (blocks > 0x7fffffffu) {
+        return TE_STATUS_UNSUPPORTED;
+    }
+    auto go = [&](auto type, auto wmc, auto g, auto gluc, auto w4c) {
+        gemm_bf16_kernel<decltype(type)::value, decltype(wmc)::value, decltype(g)::value, decltype(gluc)::value,
+                         decltype(w4c)::value>
+            <<<(unsigned)blocks, 256 * decltype(g)::value, 0, stream>>>(
+                sg, row_bytes, act_base(const_cast<void *>(act)), (int)rows, (int)k, (int)plan.per, (int)m_tiles,
+                (int)units, (int)n_tiles, part, glu_out == nullptr ? nullptr : act_base(glu_out));
+    };
+    auto with_w4 = [&](auto type, auto wmc, auto g, auto gluc) {
+        if (w4) {
+            go(type, wmc, g, gluc, std::true_type{});
+        } else {
+            go(type, wmc, g, gluc, std::false_type{});
+        }
+    };
+    auto with_glu = [&](auto type, auto wmc, auto g) {
+        if (glu) {
+            with_w4(type, wmc, g, std::true_type{});
+        } else {
+            with_w4(type, wmc, g, std::false_type{});
+        }
+    };
+    auto with_g = [&](auto type, auto wmc) {
+        if (plan.groups == 2) {
+            with_glu(type, wmc, std::integral_constant<int, 2>{});
+        } else {
+            with_glu(type, wmc, std::integral_constant<int, 1>{});
+        }
+    };
+    auto with_wm = [&](auto type) {
+        if (wm == 2) {
+            with_g(type, std::integral_constant<int, 2>{});
+        } else {
+            with_g(type, std::integral_constant<int, 4>{});
+        }
+    };
+    if (ggml_type == kQ4_0) {
+        with_wm(std::integral_constant<uint32_t, kQ4_0>{});
+    } else {
+        with_wm(std::integral_constant<uint32_t, kQ8_0>{});
+    }
+    return launch_status();
+}
+
+// Whether a tensor's rows can be read as dwords holding whole pairs of blocks.
+static bool rows_w4(const void *w, size_t row_bytes) { return ((uintptr_t)w & 3u) == 0 && row_bytes % 4 == 0; }
 
 te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, const void *act, size_t rows,
                              size_t k, float *partials, size_t partial_bytes, hipStream_t stream,
@@ -858,62 +807,27 @@ te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, 
         return TE_STATUS_UNSUPPORTED;
     }
     if (post != nullptr && nseg != 1) {
-        return TE_STATUS_INVALID_ARGUMENT;  // the digits are of one output
+        return TE_STATUS_INVALID_ARGUMENT;  // the operand is of one output
     }
     const size_t row_bytes = k / 32 * (ggml_type == kQ4_0 ? 18 : 34);
-    // the LDS-staged kernel where a row's chunks are 16-byte aligned (its
-    // split boundaries fall on whole chunks), else one gemm_q_kernel launch
-    // per matrix
-    bool staged = row_bytes % 16 == 0 && getenv("TE_HIP_GEMM_V1") == nullptr;
+    bool w4 = true;
     size_t n_total = 0, tiles_n = 0;
     for (int i = 0; i < nseg; ++i) {
         if (segs[i].n == 0 || segs[i].n > 0x7fffffffu || ((size_t)segs[i].w & 1u) != 0 ||
             (segs[i].resid != nullptr) != (segs[0].resid != nullptr)) {
             return TE_STATUS_UNSUPPORTED;
         }
-        staged = staged && ((size_t)segs[i].w & 15u) == 0;
+        w4 = w4 && rows_w4(segs[i].w, row_bytes);
         n_total += segs[i].n;
-        tiles_n += (segs[i].n + 63) / 64;
+        tiles_n += (segs[i].n + kBN - 1) / kBN;
     }
     if (n_total > 0x7fffffffu) {
         return TE_STATUS_UNSUPPORTED;
     }
-    const size_t planes = plane_bytes(rows, k);
-    const int8_t *hi = static_cast<const int8_t *>(act);
-    const int8_t *lo = hi + planes;
-    const float *scales = reinterpret_cast<const float *>(lo + planes);
-    if (!staged && nseg > 1) {
-        for (int i = 0; i < nseg; ++i) {
-            const te_status st = launch_gemm_q_segs(ggml_type, &segs[i], 1, act, rows, k, partials, partial_bytes,
-                                                    stream, nullptr);
-            if (st != TE_STATUS_OK) {
-                return st;
-            }
-        }
-        return TE_STATUS_OK;
-    }
-    const size_t tiles = tiles_n * ((rows + 63) / 64);
-    const size_t nb = k / 32;
-    // split K until the grid covers four workgroups per CU (measured: down at 512 rows 175 -> 159 us
-    // against two; eight gains nothing more), keeping >= 8 blocks per split
-    size_t splits = 1;
-    size_t per_cu = 4;
-    if (const char *env = getenv("TE_HIP_GEMM_SPLIT_TARGET")) {  // tuning override: workgroups per CU
-        const long v = strtol(env, nullptr, 10);
-        per_cu = v >= 1 && v <= 16 ? (size_t)v : per_cu;
-    }
-    const size_t want = per_cu * (size_t)device_compute_units();
-    while (partials != nullptr && tiles * splits < want && nb / (splits * 2) >= 8 &&
-           splits * 2 * rows * n_total * sizeof(float) <= partial_bytes) {
-        splits *= 2;
-    }
-    int per = (int)((nb + splits - 1) / splits);
-    if (staged) {
-        per = (per + kWChunk - 1) / kWChunk * kWChunk;
-        splits = (nb + (size_t)per - 1) / (size_t)per;
-    }
-    const dim3 grid((unsigned)tiles_n, (unsigned)((rows + 63) / 64), (unsigned)splits);
-    const bool resid = segs[0].resid != nullptr;
+    const size_t splits_max =
+        partials == nullptr ? 1 : std::max<size_t>(1, partial_bytes / (rows * n_total * sizeof(float)));
+    const GemmPlan plan = gemm_plan(rows, n_total, tiles_n, k / 32, splits_max);
+    const size_t splits = plan.splits;
     GemmSegsArg sg = {};
     sg.nseg = nseg;
     int tile_end = 0;
@@ -922,42 +836,22 @@ te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, 
         sg.out[i] = segs[i].out;
         sg.resid[i] = segs[i].resid;
         sg.n[i] = (int)segs[i].n;
-        tile_end += (int)((segs[i].n + 63) / 64);
+        tile_end += (int)((segs[i].n + kBN - 1) / kBN);
         sg.tile_end[i] = tile_end;
         sg.n_off[i + 1] = sg.n_off[i] + (int)segs[i].n;
     }
-    const unsigned char *w = sg.w[0];
     const size_t n = segs[0].n;
     float *out = segs[0].out;
     const float *res = segs[0].resid;
-#define TE_GEMM(T, R)                                                                                              \
-    do {                                                                                                           \
-        if (staged) {                                                                                              \
-            gemm_q2_kernel<T, R, false><<<grid, 256, 0, stream>>>(sg, row_bytes, hi, lo, scales, (int)rows,       \
-                                                                  (int)k, per, partials, GluDigits{});             \
-        } else {                                                                                                   \
-            gemm_q_kernel<T, R><<<grid, 256, 0, stream>>>(w, row_bytes, hi, lo, scales, (int)rows, (int)n, (int)k, \
-                                                          per, out, res, partials);                                \
-        }                                                                                                          \
-    } while (0)
-    if (ggml_type == kQ4_0) {
-        if (resid) {
-            TE_GEMM(kQ4_0, true);
-        } else {
-            TE_GEMM(kQ4_0, false);
-        }
-    } else {
-        if (resid) {
-            TE_GEMM(kQ8_0, true);
-        } else {
-            TE_GEMM(kQ8_0, false);
-        }
+    te_status st = launch_tiles(ggml_type, false, w4, sg, row_bytes, act, rows, k, plan, tiles_n, partials,
+                                nullptr, stream);
+    if (st != TE_STATUS_OK) {
+        return st;
     }
-#undef TE_GEMM
-    // the RMSNorm digits of a single output: fused into the split-K sums
+    // the RMSNorm operand of a single output: fused into the split-K sums
     // where the row fits the fused kernel, else from out afterwards
     const bool rms = post != nullptr && nseg == 1 && n % 32 == 0;
-    bool digits_done = false;
+    bool rms_done = false;
     if (splits > 1) {
         const size_t count = rows * n_total;
         bool vec = aligned16(partials) && count % 4 == 0;
@@ -968,14 +862,10 @@ te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, 
         const unsigned blocks = (unsigned)std::min<size_t>((count / width + 255) / 256, 4096);
         const char *env = getenv("TE_HIP_GEMM_REDUCE_RMS");
         if (rms && n <= (size_t)kActPass && splits <= (size_t)kRmsSplits && !(env != nullptr && env[0] == '0')) {
-            const size_t planes_out = plane_bytes(rows, n);
-            int8_t *ohi = static_cast<int8_t *>(post->act_out);
-            int8_t *olo = ohi + planes_out;
-            float *osc = reinterpret_cast<float *>(olo + planes_out);
             gemm_reduce_rms_kernel<<<(unsigned)rows, kActThreads, 0, stream>>>(
-                partials, (int)splits, count, res, out, (int)n, post->norm_w, post->eps, ohi, olo, osc,
-                vec && aligned16(post->norm_w) && aligned16(post->act_out));
-            digits_done = true;
+                partials, (int)splits, count, res, out, (int)n, post->norm_w, post->eps, act_base(post->act_out),
+                vec && aligned16(post->norm_w));
+            rms_done = true;
         } else if (nseg == 1) {
             if (vec) {
                 gemm_reduce_kernel<4><<<blocks, 256, 0, stream>>>(partials, (int)splits, count, res, out);
@@ -987,10 +877,10 @@ te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, 
         } else {
             gemm_reduce_segs_kernel<1><<<blocks, 256, 0, stream>>>(partials, (int)splits, (int)rows, sg);
         }
+        st = launch_status();
     }
-    te_status st = launch_status();
-    if (st == TE_STATUS_OK && post != nullptr && !digits_done) {
-        st = launch_quant_act(kActRmsNorm, out, nullptr, post->norm_w, post->eps, rows, n, post->act_out, stream);
+    if (st == TE_STATUS_OK && post != nullptr && !rms_done) {
+        st = launch_split_act(kActRmsNorm, out, nullptr, post->norm_w, post->eps, rows, n, post->act_out, stream);
     }
     return st;
 }
@@ -1013,42 +903,28 @@ te_status launch_gemm_glu_q(uint32_t ggml_type, const void *gate_w, const void *
                             size_t n, size_t k, void *act_out, hipStream_t stream, bool *launched) {
     *launched = false;
     const size_t row_bytes = k / 32 * (ggml_type == kQ4_0 ? 18 : 34);
-    const size_t tiles = n / 32 * ((rows + 63) / 64);
+    const size_t n_tiles = (n + kBN / 2 - 1) / (kBN / 2);
+    const size_t tiles = n_tiles * ((rows + 127) / 128);
     const char *env = getenv("TE_HIP_GEMM_GLU");
     if ((ggml_type != kQ4_0 && ggml_type != kQ8_0) || k % 32 != 0 || n % 32 != 0 || rows == 0 ||
-        rows > 0x7fffffffu || n > 0x7fffffffu || k > (1u << 24) || row_bytes % 16 != 0 ||
-        ((size_t)gate_w & 15u) != 0 || ((size_t)up_w & 15u) != 0 || getenv("TE_HIP_GEMM_V1") != nullptr ||
-        (env != nullptr && env[0] == '0') ||
-        (tiles < (size_t)device_compute_units() && !(env != nullptr && env[0] == '1'))) {
-        return TE_STATUS_OK;  // not launched: the caller runs the two GEMMs and the SwiGLU digits
+        rows > 0x7fffffffu || n > 0x7fffffffu || k > (1u << 24) || ((size_t)gate_w & 1u) != 0 ||
+        ((size_t)up_w & 1u) != 0 || (env != nullptr && env[0] == '0') ||
+        (tiles < (size_t)device_compute_units() / 2 && !(env != nullptr && env[0] == '1'))) {
+        return TE_STATUS_OK;  // not launched: the caller runs the two GEMMs and the SwiGLU operand
     }
-    const size_t planes = plane_bytes(rows, k);
-    const int8_t *hi = static_cast<const int8_t *>(act);
-    const int8_t *lo = hi + planes;
-    const float *scales = reinterpret_cast<const float *>(lo + planes);
-    const size_t out_planes = plane_bytes(rows, n);
-    GluDigits d;
-    d.hi = static_cast<int8_t *>(act_out);
-    d.lo = d.hi + out_planes;
-    d.scales = reinterpret_cast<float *>(d.lo + out_planes);
     GemmSegsArg sg = {};
     sg.nseg = 1;
     sg.w[0] = static_cast<const unsigned char *>(gate_w);
     sg.w[1] = static_cast<const unsigned char *>(up_w);
     sg.n[0] = (int)n;
-    sg.tile_end[0] = (int)(n / 32);
+    sg.tile_end[0] = (int)n_tiles;
     sg.n_off[1] = (int)n;
-    const dim3 grid((unsigned)(n / 32), (unsigned)((rows + 63) / 64), 1);
-    const int per = (int)(k / 32);
-    if (ggml_type == kQ4_0) {
-        gemm_q2_kernel<kQ4_0, false, true><<<grid, 256, 0, stream>>>(sg, row_bytes, hi, lo, scales, (int)rows, (int)k,
-                                                                     per, nullptr, d);
-    } else {
-        gemm_q2_kernel<kQ8_0, false, true><<<grid, 256, 0, stream>>>(sg, row_bytes, hi, lo, scales, (int)rows, (int)k,
-                                                                     per, nullptr, d);
-    }
+    const bool w4 = rows_w4(gate_w, row_bytes) && rows_w4(up_w, row_bytes);
+    GemmPlan plan = gemm_plan(rows, n, n_tiles, k / 32, 1);
+    // one projection's groups: the sums are those of the two GEMMs, bit for bit
+    plan.groups = gemm_plan(rows, n, (n + kBN - 1) / kBN, k / 32, 1).groups;
     *launched = true;
-    return launch_status();
+    return launch_tiles(ggml_type, true, w4, sg, row_bytes, act, rows, k, plan, n_tiles, nullptr, act_out, stream);
 }
 
 }  // namespace te_hip
@@ -1068,7 +944,7 @@ extern "C" te_status te_hip_gemm_q_f32(const void *weights, uint32_t ggml_type, 
         return TE_STATUS_INVALID_ARGUMENT;
     }
     hipStream_t s = te_hip::as_stream(stream);
-    te_status st = te_hip::launch_quant_act(pre, x, x2, norm_w, epsilon, rows, k, act, s);
+    te_status st = te_hip::launch_split_act(pre, x, x2, norm_w, epsilon, rows, k, act, s);
     if (st != TE_STATUS_OK) {
         return st;
     }

@@ -115,17 +115,14 @@ te_status launch_dequant_row(const void *weights, uint32_t ggml_type, size_t col
 te_status launch_dequant_rows(const void *weights, uint32_t ggml_type, size_t cols, const uint32_t *rows, size_t n,
                               float *out, hipStream_t stream);
 
-// Batched-prefill GEMM (te_gemm.hip).  launch_quant_act turns rows x cols fp32
+// Batched-prefill GEMM (te_gemm.hip).  launch_split_act turns rows x cols fp32
 // activations (after pre-op 0 none, 1 RMSNorm with norm_w / eps, 2 SwiGLU
-// with x2 as `up`) into the digit planes + block scales held in `act`
-// (act_buffer_bytes(rows, cols) bytes); launch_gemm_q then writes
+// with x2 as `up`) into the GEMM's operand (hi + lo bf16, te_act_split.h) held
+// in `act` (act_buffer_bytes(rows, cols) bytes); launch_gemm_q then writes
 // out[m][n] = sum_k act[m][k] W[n][k] (+ resid[m][n]) for a Q4_0 / Q8_0
 // weight tensor W [n][k] at a 2-byte aligned address.
 size_t act_buffer_bytes(size_t rows, size_t cols);
-// The layout inside `act`: the hi plane at act, the lo plane at
-// act + act_plane_bytes(rows, cols), the fp32 block scales after the lo plane.
-size_t act_plane_bytes(size_t rows, size_t cols);
-te_status launch_quant_act(int pre, const float *x, const float *x2, const float *norm_w, float eps, size_t rows,
+te_status launch_split_act(int pre, const float *x, const float *x2, const float *norm_w, float eps, size_t rows,
                            size_t cols, void *act, hipStream_t stream);
 // `partials` (partial_bytes, may be NULL) lets small output grids split K.
 te_status launch_gemm_q(const void *weights, uint32_t ggml_type, const void *act, size_t rows, size_t n, size_t k,
@@ -141,8 +138,8 @@ struct GemmSeg {
     const float *resid;
     size_t n;
 };
-// With `post` (one segment): afterwards also the RMSNorm digits of out
-// (launch_quant_act(1, out, nullptr, norm_w, eps) into act_out, the same
+// With `post` (one segment): afterwards also the RMSNorm operand of out
+// (launch_split_act(1, out, nullptr, norm_w, eps) into act_out, the same
 // bits), fused into the split-K sums where they run (TE_HIP_GEMM_REDUCE_RMS=0:
 // separate launches).  act_out may be act.
 struct GemmRmsDigits {
@@ -153,24 +150,24 @@ struct GemmRmsDigits {
 te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, const void *act, size_t rows,
                              size_t k, float *partials, size_t partial_bytes, hipStream_t stream,
                              const GemmRmsDigits *post = nullptr);
-// launch_gemm_q, then the RMSNorm digits of out (see GemmRmsDigits).
+// launch_gemm_q, then the RMSNorm operand of out (see GemmRmsDigits).
 te_status launch_gemm_q_rms(const void *weights, uint32_t ggml_type, const void *act, size_t rows, size_t n,
                             size_t k, float *out, const float *resid, float *partials, size_t partial_bytes,
                             const float *norm_w, float eps, void *act_out, hipStream_t stream);
-// Gate and up [n][k] against the same activation digits in one launch whose
-// tiles pair the same rows of both, writing silu(gate) * up as the down
-// projection's digits into act_out (act_buffer_bytes(rows, n) bytes, the same
-// digits launch_quant_act(2, gate, up) gives).  *launched = false (and
+// Gate and up [n][k] against the same activations in one launch whose tiles
+// pair the same rows of both, writing silu(gate) * up as the down projection's
+// operand into act_out (act_buffer_bytes(rows, n) bytes, the same bits
+// launch_split_act(2, gate, up) gives).  *launched = false (and
 // nothing queued) where the shapes or alignment do not allow it, n % 32 != 0,
 // or the grid would not cover the GPU: the caller then runs the two GEMMs and
-// launch_quant_act.  TE_HIP_GEMM_GLU=0 turns it off, =1 takes it for grids of
+// launch_split_act.  TE_HIP_GEMM_GLU=0 turns it off, =1 takes it for grids of
 // any size.
 te_status launch_gemm_glu_q(uint32_t ggml_type, const void *gate_w, const void *up_w, const void *act, size_t rows,
                             size_t n, size_t k, void *act_out, hipStream_t stream, bool *launched);
 
 // te_hip_attention_prefill_step_vt_f16 (te_prefill.hip; arguments as there)
-// with the attention output as the next GEMM's digits: with act_out set, the
-// launch_quant_act(0) digits of the output rows [seqs*layers*tokens][heads *
+// with the attention output as the next GEMM's operand: with act_out set, the
+// launch_split_act(0) operand of the output rows [seqs*layers*tokens][heads *
 // head_dim] go to act_out (act_buffer_bytes of that shape), formed by the
 // attention kernel from the rows it holds, and `out` is not written.  Only
 // without a key split (workspace NULL or one split): else UNSUPPORTED.

@@ -67,6 +67,8 @@
 #include <mutex>
 #include <type_traits>
 
+#include "te_act_split.h"
+
 namespace {
 
 constexpr int BM = 128;   // query rows per tile: 4 row groups of 32
@@ -104,67 +106,26 @@ struct PrefillArgs {
     int splits;      // key splits: blockIdx.z = (seq*layers + layer) * splits + split
     float *part_o;   // splits > 1: unnormalised O per (split, seq*layer, row, head), else null
     float *part_ml;  // splits > 1: (m, l) per (split, seq*layer, row, head)
-    // one split only: the output rows as the next GEMM's digits (hi / lo
-    // planes in 32 x 32 tiles, fp32 block scales; te_gemm.hip's layout)
-    // instead of fp32 rows; null: fp32 rows to `out`
-    int8_t *dhi;
-    int8_t *dlo;
-    float *dscales;
+    // one split only: the output rows as the next GEMM's operand
+    // (te_act_split.h) instead of fp32 rows; null: fp32 rows to `out`
+    unsigned char *act;
 #ifdef TE_PREFILL_PHASES
     unsigned *phase_log;  // [workgroup][wave][kPhases]: shader-clock cycles per phase, summed
 #endif
 };
 
 // Four consecutive output values (columns col .. col + 3 of `row`, col % 4
-// == 0) as digits: the eight lanes holding one 32-value block (lanes 8j ..
-// 8j + 7, every lane of the wave taking part) share its largest magnitude,
-// then each value becomes v = 256 * hi + lo at the block's scale -- the
-// arithmetic of te_gemm.hip's quant_act_kernel<kActPlain>, so the digits are
-// the ones that kernel makes from the fp32 rows.  K = the row length (heads *
-// D); only `store` lanes write.
-__device__ __forceinline__ void store_digits4(const f32x4 &v, size_t row, int K, int col, int8_t *__restrict__ hi,
-                                              int8_t *__restrict__ lo, float *__restrict__ scales, bool store) {
-    // the eight lanes' maximum by DPP moves (no LDS round trip): lanes xor 1
-    // and xor 2 within each quad, then the half-row mirror (lane i <-> 7 - i)
-    // joins the two quads
-    float m = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0xB1, 0xF, 0xF, false)));
-    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x4E, 0xF, 0xF, false)));
-    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x141, 0xF, 0xF, false)));
-    if (!store) {
-        return;
-    }
-    int q[4] = {0, 0, 0, 0};
-    float s;
-    if (!(m <= __FLT_MAX__)) {  // inf or NaN in the block: its products are NaN
-        s = __builtin_nanf("");
-    } else if (m == 0.0f) {
-        s = 0.0f;
-    } else {
-        int E;
-        (void)frexpf(m, &E);
-        const int e = min(14 - E, 126);  // blocks below 2^-112 round towards 0
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            q[j] = (int)rintf(ldexpf(v[j], e));
-        }
-        s = ldexpf(1.0f, -e);
-    }
-    // q = 256 * hi + lo with lo in [-128, 127]: hi = (q + 128) >> 8, and lo's
-    // byte is q's low byte
-    uint32_t h = 0, l = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        h |= (uint32_t)(((q[j] + 128) >> 8) & 255) << (8 * j);
-        l |= (uint32_t)(q[j] & 255) << (8 * j);
-    }
-    const int b = col >> 5;
-    const size_t t = (((row >> 5) * (size_t)(K >> 5) + b) << 10) + ((row & 31) << 5) + (col & 31);
-    *reinterpret_cast<uint32_t *>(hi + t) = h;
-    *reinterpret_cast<uint32_t *>(lo + t) = l;
-    if ((col & 31) == 0) {
-        scales[row * (size_t)(K >> 5) + b] = s;
-    }
+// == 0) as the output projection's operand: the parts te_gemm.hip's
+// split_act_kernel<kActPlain> makes from the fp32 rows.  K = the row length
+// (heads * D).
+__device__ __forceinline__ void store_act4(const f32x4 &v, size_t row, int K, int col,
+                                           unsigned char *__restrict__ act) {
+    uint2 hi, lo;
+    split_pair(v[0], v[1], hi.x, lo.x);
+    split_pair(v[2], v[3], hi.y, lo.y);
+    const size_t o = act_off(row, K >> 5, col & ~7) + 2 * (col & 4);
+    *reinterpret_cast<uint2 *>(act + o) = hi;
+    *reinterpret_cast<uint2 *>(act + o + 2048) = lo;
 }
 
 // Phase instrumentation (a build with -DTE_PREFILL_PHASES only, see
@@ -876,12 +837,13 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_causal_f16_kernel(Prefill
             // heads * D floats)
             const int row0 = wr0 + 16 * nb;
             if constexpr (Q32) {
-                if (a.dhi != nullptr) {  // the fused step's rows as digits (uniform)
+                if (a.act != nullptr) {  // the fused step's rows as the GEMM's operand (uniform)
 #pragma unroll
                     for (int i = 0; i < NS; ++i) {
                         const int r = i * (64 / LPR) + r0;
-                        store_digits4(v[i], (size_t)sl * a.tokens + row0 + r, a.heads * D, h * D + 4 * q, a.dhi,
-                                      a.dlo, a.dscales, row0 + r < a.tokens);
+                        if (row0 + r < a.tokens) {
+                            store_act4(v[i], (size_t)sl * a.tokens + row0 + r, a.heads * D, h * D + 4 * q, a.act);
+                        }
                     }
                     return;
                 }
@@ -1267,10 +1229,12 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_rows_f16_kernel(PrefillAr
         for (int p = 1; p < nact; ++p) {
             acc += *reinterpret_cast<const f32x4 *>(&part[p][r * OPITCH + 4 * q]);
         }
-        if (a.dhi != nullptr) {  // uniform
-            store_digits4(acc, (size_t)sl * a.tokens + r0 + r, a.heads * D, h * D + 4 * q, a.dhi, a.dlo, a.dscales,
-                          r0 + r < a.tokens);
-        } else if (r0 + r < a.tokens) {
+        if (r0 + r >= a.tokens) {
+            continue;
+        }
+        if (a.act != nullptr) {  // uniform
+            store_act4(acc, (size_t)sl * a.tokens + r0 + r, a.heads * D, h * D + 4 * q, a.act);
+        } else {
             float *orow = a.out + (((size_t)sl * a.tokens + r0 + r) * a.heads + h) * D;
             __builtin_nontemporal_store(acc, reinterpret_cast<f32x4 *>(orow + 4 * q));
         }
@@ -1579,7 +1543,7 @@ te_status check_prefill_args(size_t seqs, size_t layers, size_t tokens, size_t b
 
 // The attention over V^T with `splits` key splits (workspace = the partials),
 // then the merge launch when splits > 1.  With act_out (the fused step, one
-// split only): the output rows as digits, formed in the attention kernel.
+// split only): the output rows as the GEMM's operand, formed in the attention kernel.
 te_status run_prefill(PrefillArgs a, int splits, void *partials, size_t seqs, size_t layers, size_t tokens,
                       size_t base_position, size_t context_tokens, size_t heads, size_t kv_heads, size_t head_dim,
                       float *out, hipStream_t strm, void *act_out = nullptr) {
@@ -1590,10 +1554,7 @@ te_status run_prefill(PrefillArgs a, int splits, void *partials, size_t seqs, si
         a.part_o = static_cast<float *>(partials);
         a.part_ml = a.part_o + parts * head_dim;
     } else if (act_out != nullptr) {
-        const size_t planes = te_hip::act_plane_bytes(seqs * layers * tokens, heads * head_dim);
-        a.dhi = static_cast<int8_t *>(act_out);
-        a.dlo = a.dhi + planes;
-        a.dscales = reinterpret_cast<float *>(a.dlo + planes);
+        a.act = act_base(act_out);
     }
     te_status st = launch_prefill(a, seqs, layers, tokens, base_position, context_tokens, heads, kv_heads, head_dim,
                                   strm);
@@ -1721,7 +1682,7 @@ te_status te_hip::launch_prefill_step_vt(const float *query, const float *k_new,
         return TE_STATUS_UNSUPPORTED;
     }
     if (!al16(query) || !al16(q_bias) || !al16(rope_cos) || !al16(rope_sin) || !al16(key_cache) ||
-        !al16(value_cache) || !al16(value_cache_t) || !al16(out) || !al16(workspace) || !al16(act_out)) {
+        !al16(value_cache) || !al16(value_cache_t) || !al16(out) || !al16(workspace)) {
         return TE_STATUS_UNSUPPORTED;
     }
     const int splits = splits_for(workspace, workspace_bytes, seqs, layers, tokens, base_position, heads, head_dim,
@@ -1730,7 +1691,7 @@ te_status te_hip::launch_prefill_step_vt(const float *query, const float *k_new,
         return st;
     }
     if (act_out != nullptr && splits != 1) {
-        return TE_STATUS_UNSUPPORTED;  // the digits come from the one-split kernels only
+        return TE_STATUS_UNSUPPORTED;  // the operand comes from the one-split kernels only
     }
     if (al16(k_new) && al16(v_new)) {
         // bias + RoPE + fp16 append of k / v and the chunk's V^T rows: one launch

@@ -12,15 +12,14 @@
 //   x += (silu(norm Wg^T) * (norm Wu^T)) Wd^T                     (te_swiglu_f32)
 //
 // Launches per layer (one stream, no host synchronisation): the GEMM's
-// activation digits with RMSNorm folded in, then the Q, K and V GEMMs as one
+// activation operand with RMSNorm folded in, then the Q, K and V GEMMs as one
 // segmented launch (te_gemm.hip); the fused prefill step keeping V^T (bias + RoPE + fp16
 // append into the K / V caches and V^T, then the MFMA causal attention,
-// te_prefill.hip); the digits of the attention output and the Wo GEMM with
-// the residual (and the next RMSNorm's digits in its split-K sums); gate and
-// up as one launch
-// whose epilogue writes the SwiGLU digits (else two GEMMs and the SwiGLU
-// digits); the down GEMM with the residual and the next layer's attention
-// RMSNorm digits.
+// te_prefill.hip), whose output rows leave as the next operand; the Wo GEMM with
+// the residual (and the next RMSNorm's operand in its split-K sums); gate and
+// up as one launch whose epilogue writes the SwiGLU operand (else two GEMMs and
+// the SwiGLU); the down GEMM with the residual and the next layer's attention
+// RMSNorm operand.
 //
 // Differences from the Metal slot, all device-resident: the K / V caches are
 // the HIP path's fp16 caches [layers][context_tokens][kv] plus the transposed
@@ -109,16 +108,17 @@ size_t align_up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
 
 struct ChunkBuffers {
     float *q, *k, *v, *attn, *gate, *up, *part;
-    void *act, *act_ffn;  // digits of the hidden-wide inputs; of the SwiGLU output (down's input)
+    void *act, *act_ffn;  // GEMM operand of the hidden-wide inputs; of the SwiGLU output (down's input)
     size_t part_bytes;
 };
 
 // Byte layout of the workspace, in carve-up order: the GEMM outputs, the
-// split-K partial sums (up to 8 splits of a hidden-wide output), the
-// activation digits of the hidden-wide GEMM inputs, then of down's input.
+// split-K partial sums (up to 8 splits of a hidden-wide output, 20 of a short
+// chunk, whose GEMMs have few tiles), the operand of the hidden-wide GEMM
+// inputs, then of down's input.
 size_t carve(size_t batch, size_t hidden, size_t kv, size_t ffn, unsigned char *base, ChunkBuffers *b) {
     const size_t floats[7] = {batch * hidden, batch * kv, batch * kv, batch * hidden, batch * ffn, batch * ffn,
-                              8 * batch * hidden};
+                              std::max(8 * batch, 20 * std::min<size_t>(batch, 64)) * hidden};
     float **slots[7] = {&b->q, &b->k, &b->v, &b->attn, &b->gate, &b->up, &b->part};
     size_t off = 0;
     for (int i = 0; i < 7; ++i) {
@@ -240,8 +240,8 @@ static te_status prefill_all_layers_impl(
         const te_hip::GemmSeg qkv[3] = {{m + q_offsets[l], b.q, nullptr, hidden},
                                         {m + k_offsets[l], b.k, nullptr, kv},
                                         {m + v_offsets[l], b.v, nullptr, kv}};
-        // gate and up with the SwiGLU digits in their epilogue where the
-        // shapes allow it, else both GEMMs and the SwiGLU digits
+        // gate and up with the SwiGLU operand in their epilogue where the
+        // shapes allow it, else both GEMMs and the SwiGLU operand
         bool glu = false;
         auto glu_done = [&](te_status r) {
             if (glu) {
@@ -258,18 +258,18 @@ static te_status prefill_all_layers_impl(
             te_hip::prof_mark(st, share, 3);
             return staged(r);
         };
-        // the attention RMSNorm digits of layer l > 0 came with the previous
+        // the attention RMSNorm operand of layer l > 0 came with the previous
         // layer's down projection
         if ((l == 0 && !done((stage_name = "attn_norm_digits",
-                              s = te_hip::launch_quant_act(1, out, nullptr, attn_norm_weights, epsilon, batch, hidden,
+                              s = te_hip::launch_split_act(1, out, nullptr, attn_norm_weights, epsilon, batch, hidden,
                                                            b.act, st)),
                              ew)) ||
             !qkv_done((stage_name = "qkv_proj",
                        s = te_hip::launch_gemm_q_segs(ggml_type, qkv, 3, b.act, batch, hidden, b.part, b.part_bytes,
                                                       st))) ||
             // the attention output leaves the attention kernel as the output
-            // projection's digits (TE_HIP_PREFILL_DIGITS=0: fp32 rows and a
-            // digits launch, the same bits)
+            // projection's operand (TE_HIP_PREFILL_DIGITS=0: fp32 rows and a
+            // launch that splits them, the same bits)
             !done((stage_name = "qkv_bias_rope_flash_attention_mma_vt",
                    s = te_hip::launch_prefill_step_vt(
                        b.q, b.k, b.v, q_biases + l * hidden, k_biases + l * kv, v_biases + l * kv, rope_cos, rope_sin,
@@ -279,7 +279,7 @@ static te_status prefill_all_layers_impl(
                   te_hip::kProfAttention) ||
             (!attn_digits &&
              !done((stage_name = "attn_out_digits",
-                    s = te_hip::launch_quant_act(0, b.attn, nullptr, nullptr, 0.0f, batch, hidden, b.act, st)),
+                    s = te_hip::launch_split_act(0, b.attn, nullptr, nullptr, 0.0f, batch, hidden, b.act, st)),
                    ew)) ||
             !done((stage_name = "output_proj_add_ffn_norm_digits",
                    s = te_hip::launch_gemm_q_rms(m + output_offsets[l], ggml_type, b.act, batch, hidden, hidden, out,
@@ -295,11 +295,11 @@ static te_status prefill_all_layers_impl(
                      !done((stage_name = "up_proj", s = gemm(up_offsets, ffn, hidden, b.up, nullptr)),
                            te_hip::kProfUp) ||
                      !done((stage_name = "swiglu_digits",
-                            s = te_hip::launch_quant_act(2, b.gate, b.up, nullptr, 0.0f, batch, ffn, b.act_ffn, st)),
+                            s = te_hip::launch_split_act(2, b.gate, b.up, nullptr, 0.0f, batch, ffn, b.act_ffn, st)),
                            ew))) {
             break;
         }
-        // down + residual, with the next layer's attention RMSNorm digits
+        // down + residual, with the next layer's attention RMSNorm operand
         s = l + 1 < layers
                 ? te_hip::launch_gemm_q_rms(m + down_offsets[l], ggml_type, b.act_ffn, batch, hidden, ffn, out, out,
                                             b.part, b.part_bytes, attn_norm_weights + (l + 1) * hidden, epsilon,
