@@ -74,10 +74,13 @@ struct DecodeArgs {
     int heads;
     int kv_heads;
     int group;
-    int chunk;
+    int seqs;
     int max_chunks;
     float qscale;    // log2(e)/sqrt(D)
     int positions[TE_HIP_MAX_SEQS];
+    // sequence s has chunks first[s] .. first[s + 1] - 1 of the launch's list
+    // (grid.x), of ceil(tiles / chunks) tiles each
+    int first[TE_HIP_MAX_SEQS + 1];
 };
 
 template <int D>
@@ -277,18 +280,23 @@ __global__ __launch_bounds__(64, 2) void decode_splitk_f16_kernel(DecodeArgs a) 
     constexpr int NT = D / 16;  // output tiles over head_dim; also dims per lane in V loads
     constexpr int KK = D / 32;  // MFMA K-steps over head_dim for QK^T
 
-    const int chunk_id = blockIdx.x;
-    const int kvh = blockIdx.y;
-    const int sl = blockIdx.z;
-    const int s = sl / a.layers;
-    const int pos = a.positions[s];
-    const int c0 = chunk_id * a.chunk;
-    if (c0 > pos) {
-        return;  // this sequence has fewer chunks than the longest one
-    }
-    const int c1 = min(c0 + a.chunk, pos + 1);
-    const int last = c1 - 1;  // loads are clamped to the chunk; positions > pos are masked
     const int lane = threadIdx.x;
+    const int kvh = blockIdx.y;
+    // the chunk's sequence: lane i compares the end of sequence i's chunks
+    int s = 0;
+    if (a.seqs > 1) {
+        const bool past = lane < a.seqs - 1 && a.first[lane + 1] <= (int)blockIdx.x;
+        s = __builtin_amdgcn_readfirstlane(__builtin_popcountll(__builtin_amdgcn_ballot_w64(past)));
+    }
+    const int chunk_id = (int)blockIdx.x - a.first[s];
+    const int sl = s * a.layers + (int)blockIdx.z;
+    const int pos = a.positions[s];
+    const int n_chunks = a.first[s + 1] - a.first[s];
+    // (n_chunks = ceil(tiles / t) for some t, so no chunk is empty)
+    const int chunk = ((pos + kTile) / kTile + n_chunks - 1) / n_chunks * kTile;
+    const int c0 = chunk_id * chunk;
+    const int c1 = min(c0 + chunk, pos + 1);
+    const int last = c1 - 1;  // loads are clamped to the chunk; positions > pos are masked
     const int g = lane >> 4;
     const int c = lane & 15;
 
@@ -401,9 +409,8 @@ struct CombineArgs {
     int layers;
     int heads;
     int head_dim;
-    int chunk;
     int max_chunks;
-    int positions[TE_HIP_MAX_SEQS];
+    int chunks[TE_HIP_MAX_SEQS];  // of each sequence
 };
 
 // Merge of two softmax partials (m, l, o) in the log2 domain; a side whose max
@@ -433,7 +440,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(CombineArgs a) {
     const int h = blockIdx.x;
     const int sl = blockIdx.y;
     const int s = sl / a.layers;
-    const int n_chunks = (a.positions[s] + a.chunk) / a.chunk;  // ceil((pos+1)/chunk)
+    const int n_chunks = a.chunks[s];
     const size_t base = ((size_t)sl * a.heads + h) * a.max_chunks;
     const int tid = threadIdx.x;
     const int col = tid % COLS;
@@ -479,7 +486,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgs a) {
     const int h = blockIdx.x;
     const int sl = blockIdx.y;
     const int s = sl / a.layers;
-    const int n_chunks = (a.positions[s] + a.chunk) / a.chunk;  // ceil((pos+1)/chunk)
+    const int n_chunks = a.chunks[s];
     const size_t base = ((size_t)sl * a.heads + h) * a.max_chunks;
     const float *ml = a.part_ml + base * 2;
     const int tid = threadIdx.x;
@@ -614,6 +621,11 @@ bool valid_positions(const size_t *positions, size_t position, size_t seqs, size
     return true;
 }
 
+// Chunks of a sequence whose query is at `position`.
+size_t chunks_of(size_t position, const te_hip::DecodeGeometry &g) {
+    return (position + (size_t)g.chunk) / (size_t)g.chunk;
+}
+
 te_status check_decode_args(const size_t *positions, size_t position, size_t seqs, size_t layers,
                             size_t context_tokens, size_t heads, size_t kv_heads, size_t head_dim,
                             size_t *max_position) {
@@ -649,8 +661,10 @@ int device_compute_units() {
     return cus;
 }
 
+constexpr size_t kBatchChunks = 8;
+
 DecodeGeometry decode_geometry(const size_t *positions, size_t position, size_t seqs, size_t layers,
-                               size_t kv_heads) {
+                               size_t kv_heads, size_t refine_chunks) {
     // The chunk is the total number of 32-position tiles over all (seq,
     // layer, kv_head) streams divided by a target of 3.5 single-wave
     // workgroups per CU (at least two tiles, so the prefetch pipeline has
@@ -688,6 +702,20 @@ DecodeGeometry decode_geometry(const size_t *positions, size_t position, size_t 
     tiles = (max_tiles + n_longest - 1) / n_longest;           // equal chunks for it
     if (tiles < min_tiles) {
         tiles = min_tiles;
+    }
+    // A batch: the longest sequence gets at least kBatchChunks chunks (of 8
+    // tiles or more, within the chunk bound, so the workspace stays as it
+    // is).  With one to three chunks per sequence their lengths differ by
+    // several times and the long ones run on alone: 7B, 8 ragged sequences of
+    // 1.5K-16K, 28 layers 707 us with 3 chunks of the longest, 655 with 4, 609
+    // with 6, 616 with 8; 3B, 4 ragged of 73-31K 464 and 440 us; a single
+    // sequence's chunks are equal, and there finer ones cost 2-8 %.
+    if (seqs > 1) {
+        const size_t n = std::min(std::min(std::min(kBatchChunks, refine_chunks), (max_tiles + 7) / 8),
+                                  decode_chunks_bound(max_n - 1, layers, kv_heads));
+        if (n > 0) {
+            tiles = std::min(tiles, (max_tiles + n - 1) / n);
+        }
     }
     size_t chunk = tiles * kTile;
     const char *env = getenv("TE_HIP_DECODE_CHUNK");
@@ -768,9 +796,8 @@ te_status launch_decode_f32(const float *query, const float *key_cache, const fl
     c.layers = 1;
     c.heads = (int)heads;
     c.head_dim = (int)head_dim;
-    c.chunk = chunk;
     c.max_chunks = max_chunks;
-    c.positions[0] = (int)position;
+    c.chunks[0] = max_chunks;
     decode_combine_kernel<<<dim3((unsigned)heads, 1), 256, 0, stream>>>(c);
     return launch_status();
 }
@@ -827,7 +854,7 @@ namespace {
 te_status launch_splitk(const DecodeArgs &fused, bool is_fused, const float *query, const uint16_t *key_cache,
                         const uint16_t *value_cache, const size_t *positions, size_t position, size_t seqs,
                         size_t layers, size_t context_tokens, size_t heads, size_t kv_heads, size_t head_dim,
-                        void *workspace, size_t workspace_bytes, void *stream) {
+                        void *workspace, size_t workspace_bytes, void *stream, size_t refine_chunks = SIZE_MAX) {
     if (query == nullptr || key_cache == nullptr || value_cache == nullptr || workspace == nullptr) {
         return TE_STATUS_INVALID_ARGUMENT;
     }
@@ -837,7 +864,8 @@ te_status launch_splitk(const DecodeArgs &fused, bool is_fused, const float *que
     if (st != TE_STATUS_OK) {
         return st;
     }
-    const te_hip::DecodeGeometry geo = te_hip::decode_geometry(positions, position, seqs, layers, kv_heads);
+    const te_hip::DecodeGeometry geo =
+        te_hip::decode_geometry(positions, position, seqs, layers, kv_heads, refine_chunks);
     if (workspace_bytes < te_hip::decode_workspace_bytes(geo, seqs, layers, heads, head_dim)) {
         return TE_STATUS_INVALID_ARGUMENT;
     }
@@ -853,13 +881,14 @@ te_status launch_splitk(const DecodeArgs &fused, bool is_fused, const float *que
     a.heads = (int)heads;
     a.kv_heads = (int)kv_heads;
     a.group = (int)(heads / kv_heads);
-    a.chunk = geo.chunk;
+    a.seqs = (int)seqs;
     a.max_chunks = geo.max_chunks;
     a.qscale = TE_LOG2E / sqrtf((float)head_dim);
     for (size_t s = 0; s < seqs; ++s) {
         a.positions[s] = (int)(positions != nullptr ? positions[s] : position);
+        a.first[s + 1] = a.first[s] + (int)chunks_of((size_t)a.positions[s], geo);
     }
-    const dim3 grid((unsigned)geo.max_chunks, (unsigned)kv_heads, (unsigned)(seqs * layers));
+    const dim3 grid((unsigned)a.first[seqs], (unsigned)kv_heads, (unsigned)layers);
     hipStream_t strm = te_hip::as_stream(stream);
     if (head_dim == 128) {
         if (is_fused) {
@@ -890,15 +919,14 @@ extern "C" te_status te_hip_attention_decode_splitk_f16(
                          context_tokens, heads, kv_heads, head_dim, workspace, workspace_bytes, stream);
 }
 
-extern "C" te_status te_hip_attention_decode_step_splitk_f16(
-    const float *query, const float *k_new, const float *v_new,
-    const float *q_bias, const float *k_bias, const float *v_bias,
-    const float *rope_cos, const float *rope_sin,
-    uint16_t *key_cache, uint16_t *value_cache,
-    const size_t *positions, size_t position,
-    size_t seqs, size_t layers, size_t context_tokens,
-    size_t heads, size_t kv_heads, size_t head_dim,
-    void *workspace, size_t workspace_bytes, void *stream) {
+namespace {
+
+te_status step_splitk(const float *query, const float *k_new, const float *v_new, const float *q_bias,
+                      const float *k_bias, const float *v_bias, const float *rope_cos, const float *rope_sin,
+                      uint16_t *key_cache, uint16_t *value_cache, const size_t *positions, size_t position,
+                      size_t seqs, size_t layers, size_t context_tokens, size_t heads, size_t kv_heads,
+                      size_t head_dim, void *workspace, size_t workspace_bytes, void *stream,
+                      size_t refine_chunks) {
     if (k_new == nullptr || v_new == nullptr || rope_cos == nullptr || rope_sin == nullptr) {
         return TE_STATUS_INVALID_ARGUMENT;
     }
@@ -913,7 +941,28 @@ extern "C" te_status te_hip_attention_decode_step_splitk_f16(
     f.key_cache_w = reinterpret_cast<f16 *>(key_cache);
     f.value_cache_w = reinterpret_cast<f16 *>(value_cache);
     return launch_splitk(f, true, query, key_cache, value_cache, positions, position, seqs, layers,
-                         context_tokens, heads, kv_heads, head_dim, workspace, workspace_bytes, stream);
+                         context_tokens, heads, kv_heads, head_dim, workspace, workspace_bytes, stream,
+                         refine_chunks);
+}
+
+te_status launch_combine(const size_t *positions, size_t position, size_t seqs, size_t layers, size_t heads,
+                         size_t kv_heads, size_t head_dim, float *out, const void *workspace,
+                         size_t workspace_bytes, void *stream, size_t refine_chunks);
+
+}  // namespace
+
+extern "C" te_status te_hip_attention_decode_step_splitk_f16(
+    const float *query, const float *k_new, const float *v_new,
+    const float *q_bias, const float *k_bias, const float *v_bias,
+    const float *rope_cos, const float *rope_sin,
+    uint16_t *key_cache, uint16_t *value_cache,
+    const size_t *positions, size_t position,
+    size_t seqs, size_t layers, size_t context_tokens,
+    size_t heads, size_t kv_heads, size_t head_dim,
+    void *workspace, size_t workspace_bytes, void *stream) {
+    return step_splitk(query, k_new, v_new, q_bias, k_bias, v_bias, rope_cos, rope_sin, key_cache, value_cache,
+                       positions, position, seqs, layers, context_tokens, heads, kv_heads, head_dim, workspace,
+                       workspace_bytes, stream, SIZE_MAX);
 }
 
 extern "C" te_status te_hip_attention_decode_step_f16(
@@ -938,10 +987,11 @@ extern "C" te_status te_hip_attention_decode_step_f16(
                                            workspace, workspace_bytes, stream);
 }
 
-extern "C" te_status te_hip_attention_decode_combine(
-    const size_t *positions, size_t position,
-    size_t seqs, size_t layers, size_t heads, size_t kv_heads, size_t head_dim,
-    float *out, const void *workspace, size_t workspace_bytes, void *stream) {
+namespace {
+
+te_status launch_combine(const size_t *positions, size_t position, size_t seqs, size_t layers, size_t heads,
+                         size_t kv_heads, size_t head_dim, float *out, const void *workspace,
+                         size_t workspace_bytes, void *stream, size_t refine_chunks) {
     if (out == nullptr || workspace == nullptr) {
         return TE_STATUS_INVALID_ARGUMENT;
     }
@@ -957,7 +1007,8 @@ extern "C" te_status te_hip_attention_decode_combine(
     if (st != TE_STATUS_OK) {
         return st;
     }
-    const te_hip::DecodeGeometry geo = te_hip::decode_geometry(positions, position, seqs, layers, kv_heads);
+    const te_hip::DecodeGeometry geo =
+        te_hip::decode_geometry(positions, position, seqs, layers, kv_heads, refine_chunks);
     if (workspace_bytes < te_hip::decode_workspace_bytes(geo, seqs, layers, heads, head_dim)) {
         return TE_STATUS_INVALID_ARGUMENT;
     }
@@ -969,10 +1020,9 @@ extern "C" te_status te_hip_attention_decode_combine(
     c.layers = (int)layers;
     c.heads = (int)heads;
     c.head_dim = (int)head_dim;
-    c.chunk = geo.chunk;
     c.max_chunks = geo.max_chunks;
     for (size_t s = 0; s < seqs; ++s) {
-        c.positions[s] = (int)(positions != nullptr ? positions[s] : position);
+        c.chunks[s] = (int)chunks_of(positions != nullptr ? positions[s] : position, geo);
     }
     const dim3 grid((unsigned)heads, (unsigned)(seqs * layers));
     if (head_dim == 128) {
@@ -981,6 +1031,16 @@ extern "C" te_status te_hip_attention_decode_combine(
         decode_merge_kernel<64><<<grid, 256, 0, te_hip::as_stream(stream)>>>(c);
     }
     return te_hip::launch_status();
+}
+
+}  // namespace
+
+extern "C" te_status te_hip_attention_decode_combine(
+    const size_t *positions, size_t position,
+    size_t seqs, size_t layers, size_t heads, size_t kv_heads, size_t head_dim,
+    float *out, const void *workspace, size_t workspace_bytes, void *stream) {
+    return launch_combine(positions, position, seqs, layers, heads, kv_heads, head_dim, out, workspace,
+                          workspace_bytes, stream, SIZE_MAX);
 }
 
 // ---- te_hip_attention_decode_step_noalloc_f16 -------------------------------
@@ -1047,8 +1107,11 @@ extern "C" te_status te_hip_attention_decode_step_noalloc_f16(
         return st;
     }
     // The partials this exact call writes (not the position-monotone bound
-    // the workspace query reports) must fit the array.
-    const te_hip::DecodeGeometry geo = te_hip::decode_geometry(positions, position, seqs, layers, kv_heads);
+    // the workspace query reports) must fit the array; a batch is cut no finer
+    // than that.
+    const size_t per_chunk = te_hip::decode_workspace_bytes({0, 1}, seqs, layers, heads, head_dim);
+    const size_t refine = (size_t)TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES / per_chunk;
+    const te_hip::DecodeGeometry geo = te_hip::decode_geometry(positions, position, seqs, layers, kv_heads, refine);
     const size_t need = te_hip::decode_workspace_bytes(geo, seqs, layers, heads, head_dim);
     if (need > (size_t)TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES) {
         return TE_STATUS_UNSUPPORTED;
@@ -1057,8 +1120,12 @@ extern "C" te_status te_hip_attention_decode_step_noalloc_f16(
     if ((st = scratch_address(&ws)) != TE_STATUS_OK) {
         return st;
     }
-    return te_hip_attention_decode_step_f16(query, k_new, v_new, q_bias, k_bias, v_bias, rope_cos, rope_sin,
-                                            key_cache, value_cache, positions, position, seqs, layers,
-                                            context_tokens, heads, kv_heads, head_dim, out, ws,
-                                            (size_t)TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES, stream);
+    st = step_splitk(query, k_new, v_new, q_bias, k_bias, v_bias, rope_cos, rope_sin, key_cache, value_cache,
+                     positions, position, seqs, layers, context_tokens, heads, kv_heads, head_dim, ws,
+                     (size_t)TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES, stream, refine);
+    if (st != TE_STATUS_OK) {
+        return st;
+    }
+    return launch_combine(positions, position, seqs, layers, heads, kv_heads, head_dim, out, ws,
+                          (size_t)TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES, stream, refine);
 }

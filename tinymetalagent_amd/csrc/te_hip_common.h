@@ -78,7 +78,7 @@ inline te_status launch_status() {
 // Decode split-K geometry, shared by the split-K and combine launches and the
 // workspace-size query so all three agree.
 struct DecodeGeometry {
-    int chunk;       // cache positions per workgroup (multiple of 32)
+    int chunk;       // most cache positions per workgroup (multiple of 32)
     int max_chunks;  // chunks of the longest sequence
 };
 
@@ -217,8 +217,10 @@ te_status launch_gemv_merge(uint32_t ggml_type, const GemvSeg &seg, size_t cols,
                             const float *part_ml, size_t chunks, size_t max_chunks, size_t head_dim,
                             hipStream_t stream, bool *launched);
 
+// refine_chunks: the most chunks a batch's longest sequence is cut into for
+// balance (a geometry that needs more for its size keeps them).
 DecodeGeometry decode_geometry(const size_t *positions, size_t position, size_t seqs, size_t layers,
-                               size_t kv_heads);
+                               size_t kv_heads, size_t refine_chunks = SIZE_MAX);
 
 size_t decode_workspace_bytes(const DecodeGeometry &g, size_t seqs, size_t layers, size_t heads, size_t head_dim);
 
