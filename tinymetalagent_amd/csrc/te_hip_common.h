@@ -169,15 +169,16 @@ te_status launch_gemm_glu_q(uint32_t ggml_type, const void *gate_w, const void *
 // with the attention output as the next GEMM's operand: with act_out set, the
 // launch_split_act(0) operand of the output rows [seqs*layers*tokens][heads *
 // head_dim] go to act_out (act_buffer_bytes of that shape), formed by the
-// attention kernel from the rows it holds, and `out` is not written.  Only
-// without a key split (workspace NULL or one split): else UNSUPPORTED.
+// attention kernel (or the key splits' merge) from the rows it holds, and `out`
+// is not written.  fit_splits: as many key splits as the workspace holds
+// partials for, instead of INVALID_ARGUMENT where it is too small.
 te_status launch_prefill_step_vt(const float *query, const float *k_new, const float *v_new, const float *q_bias,
                                  const float *k_bias, const float *v_bias, const float *rope_cos,
                                  const float *rope_sin, uint16_t *key_cache, uint16_t *value_cache,
                                  uint16_t *value_cache_t, size_t seqs, size_t layers, size_t tokens,
                                  size_t base_position, size_t context_tokens, size_t heads, size_t kv_heads,
                                  size_t head_dim, float *out, void *act_out, void *workspace, size_t workspace_bytes,
-                                 hipStream_t stream);
+                                 bool fit_splits, hipStream_t stream);
 
 // One weight matrix of a fused GEMV launch: out[r] = W[r] . x' (+ resid[r] when
 // resid is set; resid may equal out), r < rows.

@@ -128,6 +128,12 @@ __device__ __forceinline__ void store_act4(const f32x4 &v, size_t row, int K, in
     *reinterpret_cast<uint2 *>(act + o + 2048) = lo;
 }
 
+// The causal kernel's forms, one instantiation each (a path that a form does
+// not take costs it registers: the fused step with both outputs in one form
+// spilled 17-20 SGPRs and ran 1-2 % slower): fp16 queries; fp32 queries with
+// bias and RoPE on load; those with the output rows as the GEMM's operand.
+enum { kQ16 = 0, kQ32 = 1, kQ32Act = 2 };
+
 // Phase instrumentation (a build with -DTE_PREFILL_PHASES only, see
 // build.py --phases and bench.py --phases): each wave sums s_memtime deltas
 // per phase of the step loop and writes them when it ends.
@@ -246,11 +252,10 @@ struct DmaPlan {
     int vsoff;
 };
 
-// Q32: the fused step's fp32 queries (bias + RoPE on load), else fp16
-// queries; one instantiation per query kind keeps each kind's registers to
-// its own path.
-template <int D, bool Q32>
+template <int D, int MODE>
 __global__ __launch_bounds__(kThreads, 1) void prefill_causal_f16_kernel(PrefillArgs a) {
+    constexpr bool Q32 = MODE != kQ16;
+
     typedef KHalf<D> KH;
     typedef VtHalf<D> VH;
     constexpr int KK = D / 32;                      // QK^T K-steps
@@ -836,17 +841,15 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_causal_f16_kernel(Prefill
             // a 32-bit float offset from the block's first row (16 rows of
             // heads * D floats)
             const int row0 = wr0 + 16 * nb;
-            if constexpr (Q32) {
-                if (a.act != nullptr) {  // the fused step's rows as the GEMM's operand (uniform)
+            if constexpr (MODE == kQ32Act) {
 #pragma unroll
-                    for (int i = 0; i < NS; ++i) {
-                        const int r = i * (64 / LPR) + r0;
-                        if (row0 + r < a.tokens) {
-                            store_act4(v[i], (size_t)sl * a.tokens + row0 + r, a.heads * D, h * D + 4 * q, a.act);
-                        }
+                for (int i = 0; i < NS; ++i) {
+                    const int r = i * (64 / LPR) + r0;
+                    if (row0 + r < a.tokens) {
+                        store_act4(v[i], (size_t)sl * a.tokens + row0 + r, a.heads * D, h * D + 4 * q, a.act);
                     }
-                    return;
                 }
+                return;
             }
             float *orow = a.out + (((size_t)sl * a.tokens + row0) * a.heads + h) * D;
             const unsigned rstride = (unsigned)a.heads * D;
@@ -1255,38 +1258,66 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_rows_f16_kernel(PrefillAr
 // Key-split merge: out[row][h] = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s
 // over the splits of one (seq*layer); M = max_s m_s.  A split that saw no
 // unmasked key of the row has m_s = -inf and weight 0 (split 0 always holds
-// key 0).  Thread (item, col) handles 4 dims of one (row, head).
+// key 0).  Thread (item, col) handles 4 dims of one (row, head); the splits'
+// loads are issued eight at a time (one by one, each split added its load's
+// latency: 64 rows after 2000 at 3B, 16 splits 13 us).  With `act`, the rows
+// leave as the output projection's operand instead of fp32.
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part_o, const float *part_ml, int splits,
-                                                           int items, float *out) {
+                                                           int items, int heads, float *out, unsigned char *act) {
     constexpr int COLS = D / 4;
     constexpr int ITEMS = 256 / COLS;
+    constexpr int B = 8;
     const int item = blockIdx.x * ITEMS + (int)threadIdx.x / COLS;
     const int col = threadIdx.x % COLS;
     if (item >= items) {
         return;
     }
     const size_t sl = blockIdx.y;
+    const size_t p0 = sl * splits * items + item;
+    const float2 *mls = reinterpret_cast<const float2 *>(part_ml) + p0;
+    const float4 *os = reinterpret_cast<const float4 *>(part_o + p0 * D) + col;
     float m = -INFINITY;
-    for (int sp = 0; sp < splits; ++sp) {
-        m = fmaxf(m, part_ml[2 * ((sl * splits + sp) * items + item)]);
+    for (int s0 = 0; s0 < splits; s0 += B) {
+        float v[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            v[j] = mls[(size_t)min(s0 + j, splits - 1) * items].x;
+        }
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            m = fmaxf(m, v[j]);
+        }
     }
     float den = 0.0f;
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int sp = 0; sp < splits; ++sp) {
-        const size_t pi = (sl * splits + sp) * items + item;
-        const float2 ml = *reinterpret_cast<const float2 *>(part_ml + 2 * pi);
-        const float w = ml.x == -INFINITY ? 0.0f : fast_exp2(ml.x - m);
-        const float4 o = reinterpret_cast<const float4 *>(part_o + pi * D)[col];
-        den += w * ml.y;
-        acc.x += w * o.x;
-        acc.y += w * o.y;
-        acc.z += w * o.z;
-        acc.w += w * o.w;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < splits; s0 += B) {
+        float2 ml[B];
+        float4 o[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const size_t at = (size_t)min(s0 + j, splits - 1) * items;
+            ml[j] = mls[at];
+            o[j] = os[at * COLS];
+        }
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            if (s0 + j < splits) {
+                const float w = ml[j].x == -INFINITY ? 0.0f : fast_exp2(ml[j].x - m);
+                den += w * ml[j].y;
+                acc[0] += w * o[j].x;
+                acc[1] += w * o[j].y;
+                acc[2] += w * o[j].z;
+                acc[3] += w * o[j].w;
+            }
+        }
     }
-    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-    reinterpret_cast<float4 *>(out + (sl * items + item) * D)[col] =
-        make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    acc *= den > 0.0f ? 1.0f / den : 0.0f;
+    if (act != nullptr) {
+        store_act4(acc, sl * (items / heads) + item / heads, heads * D, item % heads * D + 4 * col, act);
+    } else {
+        *reinterpret_cast<f32x4 *>(out + (sl * items + item) * D + 4 * col) = acc;
+    }
 }
 
 // V^T of positions [first, end) of every (seq*layer, kv head):
@@ -1457,31 +1488,36 @@ te_status launch_prefill(PrefillArgs a, size_t seqs, size_t layers, size_t token
     const int n_units_x = a.paired ? (a.n_qtiles + 1) / 2 : a.n_qtiles;
     const dim3 grid((unsigned)n_units_x, (unsigned)heads, (unsigned)(seqs * layers * a.splits));
     if (head_dim == 128) {
-        if (a.q32 != nullptr) {
-            prefill_causal_f16_kernel<128, true><<<grid, kThreads, 0, strm>>>(a);
+        if (a.act != nullptr) {
+            prefill_causal_f16_kernel<128, kQ32Act><<<grid, kThreads, 0, strm>>>(a);
+        } else if (a.q32 != nullptr) {
+            prefill_causal_f16_kernel<128, kQ32><<<grid, kThreads, 0, strm>>>(a);
         } else {
-            prefill_causal_f16_kernel<128, false><<<grid, kThreads, 0, strm>>>(a);
+            prefill_causal_f16_kernel<128, kQ16><<<grid, kThreads, 0, strm>>>(a);
         }
+    } else if (a.act != nullptr) {
+        prefill_causal_f16_kernel<64, kQ32Act><<<grid, kThreads, 0, strm>>>(a);
     } else if (a.q32 != nullptr) {
-        prefill_causal_f16_kernel<64, true><<<grid, kThreads, 0, strm>>>(a);
+        prefill_causal_f16_kernel<64, kQ32><<<grid, kThreads, 0, strm>>>(a);
     } else {
-        prefill_causal_f16_kernel<64, false><<<grid, kThreads, 0, strm>>>(a);
+        prefill_causal_f16_kernel<64, kQ16><<<grid, kThreads, 0, strm>>>(a);
     }
     return te_hip::launch_status();
 }
 
-// Key splits for a launch whose tile pairs alone leave CUs idle.  One
-// workgroup fills a CU (its LDS), every pair carries the same causal work
-// (~ the steps of tiles n-1-i and i), and a launch of W workgroups runs in
-// ceil(W / CUs) rounds, so S splits take ceil(S*W0 / CUs) * ceil(steps / S)
-// step times (a step, 128 keys for 256 rows, is ~2.5 us).  The merge costs a
-// launch (~2 steps) plus writing and reading every split's partial rows,
-// priced at 8 TB/s (fitted on MI355X over 3B L = 512..4096 and 1.5B 2K chunks
-// at bases 0..131072: it picks the fastest measured S or one within 4 %).
-// The smallest S with the least time wins; S = 1 whenever the pairs fill the
-// device.  TE_HIP_PREFILL_SPLITS (1..32) overrides the choice.
+// Key splits for a launch whose tiles alone leave CUs idle (or fill them
+// unevenly), from its estimated time.  One workgroup fills a CU (its LDS) and a
+// launch of W workgroups runs in ceil(W / CUs) rounds, each the longest unit's
+// steps (128 keys; 1.5 us on few CUs, 1.85 on all: the clock falls) and a fixed
+// part per tile; the merge is a launch and every split's partial rows written
+// and read.  Measured on MI355X, fused step with the append, S splits (u: one
+// tile per workgroup, p: pairs): 1.5B 2048 rows after 14336 219 us (1u), 247
+// (2u), 228 (2p), 226 (4u), 236 (5p); 3B 1024 after 8000 126 (1u), 95 (2u),
+// 107 (3p); 7B 700 after 5000 87 (1u), 90 (3u); 1.5B 300 after 9000 128 (1u),
+// 45 (6u); 3B 64 after 2000 37 (1u), 23 (4u).  The smallest S with the least
+// time wins.  TE_HIP_PREFILL_SPLITS (1..32) overrides the choice.
 int prefill_splits(size_t seqs, size_t layers, size_t tokens, size_t base_position, size_t heads,
-                   size_t head_dim) {
+                   size_t head_dim, size_t max_splits = kMaxPrefillSplits) {
     const size_t n_qtiles = (tokens + BM - 1) / BM;
     const size_t cus = (size_t)te_hip::device_compute_units();
     auto tile_steps = [&](size_t qt) {
@@ -1491,33 +1527,32 @@ int prefill_splits(size_t seqs, size_t layers, size_t tokens, size_t base_positi
     const char *env = getenv("TE_HIP_PREFILL_SPLITS");
     if (env != nullptr) {
         const long v = strtol(env, nullptr, 10);
-        if (v >= 1 && v <= kMaxPrefillSplits && (size_t)v * seqs * layers <= 65535) {
+        if (v >= 1 && v <= kMaxPrefillSplits && (size_t)v <= max_splits && (size_t)v * seqs * layers <= 65535) {
             return (int)v;
         }
     }
-    // A unit's time in step times: its steps split S ways, plus ~2.5 steps of
-    // prologue and merge per tile it holds; units run in ceil(S*W / CUs) rounds.
-    auto launch_steps = [&](int sp) {
-        const bool paired = prefill_paired(seqs, layers, tokens, heads, sp);
-        const size_t units = (paired ? (n_qtiles + 1) / 2 : n_qtiles) * heads * seqs * layers;
-        const size_t tiles = paired && n_qtiles > 1 ? 2 : 1;
-        const size_t steps = tile_steps(n_qtiles - 1) + (tiles > 1 ? tile_steps(0) : 0);
-        return (double)((sp * units + cus - 1) / cus) * ((double)((steps + sp - 1) / sp) + 2.5 * (double)tiles);
+    const double bytes = (double)(seqs * layers * tokens * heads * (head_dim + 2) * sizeof(float));
+    auto launch_us = [&](size_t sp) {
+        const bool paired = prefill_paired(seqs, layers, tokens, heads, (int)sp);
+        const size_t units = (paired ? (n_qtiles + 1) / 2 : n_qtiles) * heads * seqs * layers * sp;
+        const bool two = paired && n_qtiles > 1;
+        const size_t steps = tile_steps(n_qtiles - 1) + (two ? tile_steps(0) : 0);
+        const double busy = std::min(1.0, (double)units / (double)cus);
+        const double step_us = (1.5 + 0.35 * busy) * (head_dim == 64 ? 0.65 : 1.0);
+        return (double)((units + cus - 1) / cus) * ((double)((steps + sp - 1) / sp) * step_us + (two ? 11.5 : 6.5)) +
+               (sp > 1 ? 3.5 + (double)sp * (0.1 + bytes * 2.0 / 4.5e6) : 0.0);
     };
-    // partial bytes of one split, written then read, in step times
-    const double split_steps = (double)(seqs * layers * tokens * heads * (head_dim + 2) * sizeof(float)) * 2.0 /
-                               (8.0e12 * 2.5e-6);
     const size_t max_steps = tile_steps(n_qtiles - 1) + (n_qtiles > 1 ? tile_steps(0) : 0);
-    int best = 1;
-    double best_t = launch_steps(1);
-    for (int sp = 2; sp <= kMaxPrefillSplits && (size_t)sp <= max_steps; ++sp) {
-        const double t = launch_steps(sp) + 2.0 + split_steps * (double)sp;
-        if (t < best_t && (size_t)sp * seqs * layers <= 65535) {
-            best_t = t;
+    size_t best = 1;
+    double best_us = launch_us(1);
+    for (size_t sp = 2; sp <= std::min<size_t>(kMaxPrefillSplits, max_splits) && sp <= max_steps; ++sp) {
+        const double us = launch_us(sp);
+        if (us < best_us && sp * seqs * layers <= 65535) {
+            best_us = us;
             best = sp;
         }
     }
-    return best;
+    return (int)best;
 }
 
 size_t prefill_workspace(int splits, size_t seqs, size_t layers, size_t tokens, size_t heads, size_t head_dim) {
@@ -1542,8 +1577,8 @@ te_status check_prefill_args(size_t seqs, size_t layers, size_t tokens, size_t b
 }
 
 // The attention over V^T with `splits` key splits (workspace = the partials),
-// then the merge launch when splits > 1.  With act_out (the fused step, one
-// split only): the output rows as the GEMM's operand, formed in the attention kernel.
+// then the merge launch when splits > 1.  With act_out (the fused step): the
+// output rows as the GEMM's operand, formed in the last of these launches.
 te_status run_prefill(PrefillArgs a, int splits, void *partials, size_t seqs, size_t layers, size_t tokens,
                       size_t base_position, size_t context_tokens, size_t heads, size_t kv_heads, size_t head_dim,
                       float *out, hipStream_t strm, void *act_out = nullptr) {
@@ -1564,10 +1599,11 @@ te_status run_prefill(PrefillArgs a, int splits, void *partials, size_t seqs, si
     const int items = (int)(tokens * heads);
     const int per_block = 256 / (int)(head_dim / 4);
     const dim3 grid((unsigned)((items + per_block - 1) / per_block), (unsigned)(seqs * layers));
+    unsigned char *act = act_out == nullptr ? nullptr : act_base(act_out);
     if (head_dim == 128) {
-        prefill_merge_kernel<128><<<grid, 256, 0, strm>>>(a.part_o, a.part_ml, splits, items, out);
+        prefill_merge_kernel<128><<<grid, 256, 0, strm>>>(a.part_o, a.part_ml, splits, items, (int)heads, out, act);
     } else {
-        prefill_merge_kernel<64><<<grid, 256, 0, strm>>>(a.part_o, a.part_ml, splits, items, out);
+        prefill_merge_kernel<64><<<grid, 256, 0, strm>>>(a.part_o, a.part_ml, splits, items, (int)heads, out, act);
     }
     return te_hip::launch_status();
 }
@@ -1669,7 +1705,8 @@ te_status te_hip::launch_prefill_step_vt(const float *query, const float *k_new,
                                          uint16_t *value_cache, uint16_t *value_cache_t, size_t seqs, size_t layers,
                                          size_t tokens, size_t base_position, size_t context_tokens, size_t heads,
                                          size_t kv_heads, size_t head_dim, float *out, void *act_out,
-                                         void *workspace, size_t workspace_bytes, hipStream_t strm) {
+                                         void *workspace, size_t workspace_bytes, bool fit_splits,
+                                         hipStream_t strm) {
     if (query == nullptr || k_new == nullptr || v_new == nullptr || rope_cos == nullptr || rope_sin == nullptr ||
         key_cache == nullptr || value_cache == nullptr || value_cache_t == nullptr || out == nullptr) {
         return TE_STATUS_INVALID_ARGUMENT;
@@ -1685,13 +1722,14 @@ te_status te_hip::launch_prefill_step_vt(const float *query, const float *k_new,
         !al16(value_cache) || !al16(value_cache_t) || !al16(out) || !al16(workspace)) {
         return TE_STATUS_UNSUPPORTED;
     }
-    const int splits = splits_for(workspace, workspace_bytes, seqs, layers, tokens, base_position, heads, head_dim,
-                                  &st);
+    // the layer flow's workspace holds what it holds; a caller's has to fit
+    const int splits =
+        fit_splits ? prefill_splits(seqs, layers, tokens, base_position, heads, head_dim,
+                                    std::max<size_t>(1, 2 * workspace_bytes / prefill_workspace(2, seqs, layers, tokens,
+                                                                                                heads, head_dim)))
+                   : splits_for(workspace, workspace_bytes, seqs, layers, tokens, base_position, heads, head_dim, &st);
     if (st != TE_STATUS_OK) {
         return st;
-    }
-    if (act_out != nullptr && splits != 1) {
-        return TE_STATUS_UNSUPPORTED;  // the operand comes from the one-split kernels only
     }
     if (al16(k_new) && al16(v_new)) {
         // bias + RoPE + fp16 append of k / v and the chunk's V^T rows: one launch
@@ -1734,7 +1772,7 @@ extern "C" te_status te_hip_attention_prefill_step_vt_f16(
     return te_hip::launch_prefill_step_vt(query, k_new, v_new, q_bias, k_bias, v_bias, rope_cos, rope_sin, key_cache,
                                           value_cache, value_cache_t, seqs, layers, tokens, base_position,
                                           context_tokens, heads, kv_heads, head_dim, out, nullptr, workspace,
-                                          workspace_bytes, te_hip::as_stream(stream));
+                                          workspace_bytes, false, te_hip::as_stream(stream));
 }
 
 // ---- entry points over the plain value cache: V^T is built per call --------

@@ -275,7 +275,7 @@ static te_status prefill_all_layers_impl(
                        b.q, b.k, b.v, q_biases + l * hidden, k_biases + l * kv, v_biases + l * kv, rope_cos, rope_sin,
                        key_cache + l * ctx_kv, value_cache + l * ctx_kv, value_cache_t + l * vt_layer, 1, 1, batch,
                        base_position, context_tokens, heads, kv_heads, head_dim, b.attn, attn_digits ? b.act : nullptr,
-                       nullptr, 0, st)),
+                       b.part, b.part_bytes, true, st)),
                   te_hip::kProfAttention) ||
             (!attn_digits &&
              !done((stage_name = "attn_out_digits",
