@@ -158,10 +158,6 @@ static te_status decode_all_layers_impl(
 
     const hipStream_t st = te_hip::as_stream(stream);
     te_hip::prof_begin(st);
-    if (out != hidden_in && hipMemcpyAsync(out, hidden_in, hidden * sizeof(float), hipMemcpyDeviceToDevice, st) !=
-                                hipSuccess) {
-        return TE_STATUS_RUNTIME_ERROR;
-    }
     using te_hip::prof_mark;
     const te_hip::ProfShare qkv_share[3] = {
         {te_hip::kProfQ, (double)hidden}, {te_hip::kProfK, (double)kv}, {te_hip::kProfV, (double)kv}};
@@ -185,14 +181,16 @@ static te_status decode_all_layers_impl(
         const te_hip::GemvSeg qkv[3] = {{m + q_offsets[l], b.q, nullptr, hidden},
                                         {m + k_offsets[l], b.k, nullptr, kv},
                                         {m + v_offsets[l], b.v, nullptr, kv}};
-        s = te_hip::launch_gemv(ggml_type, te_hip::kGemvRmsNorm, qkv, 3, hidden, out, nullptr,
+        // the first layer reads hidden_in itself (a copy to out took a launch)
+        const float *x = l == 0 ? hidden_in : out;
+        s = te_hip::launch_gemv(ggml_type, te_hip::kGemvRmsNorm, qkv, 3, hidden, x, nullptr,
                                 attn_norm_weights + l * hidden, epsilon, b.xtmp, b.proj, st);
         if (s != TE_STATUS_OK) {
             break;
         }
         prof_mark(st, qkv_share, 3);
         const size_t cache_off = l * context_tokens * kv;
-        const te_hip::GemvSeg o = {m + output_offsets[l], out, out, hidden};
+        const te_hip::GemvSeg o = {m + output_offsets[l], out, x, hidden};
         bool merged_in_wo = false;
         if (merge_wo) {
             s = te_hip_attention_decode_step_splitk_f16(b.q, b.k, b.v, q_biases + l * hidden, k_biases + l * kv,

@@ -100,8 +100,9 @@ te_status library_buffer(LibraryBuffer which, size_t bytes, void **ptr);
 
 // Decode-layer vector operations (te_vecops.hip); arguments already checked.
 size_t ggml_row_bytes(uint32_t ggml_type, size_t cols);  // 0 = type / cols not supported
+// (resid, may be out: added; only where the launch can, see matvec_adds)
 te_status launch_matvec(const void *weights, uint32_t ggml_type, const float *input, size_t cols, size_t rows,
-                        float *out, hipStream_t stream);
+                        float *out, hipStream_t stream, const float *resid = nullptr);
 te_status launch_rmsnorm(const float *input, const float *weight, size_t rows, size_t len, float epsilon, float *out,
                          hipStream_t stream);
 te_status launch_swiglu(const float *gate, const float *up, size_t len, float *out, hipStream_t stream);

@@ -204,10 +204,6 @@ static te_status prefill_all_layers_impl(
     const hipStream_t st = te_hip::as_stream(stream);
     const char *digits_env = getenv("TE_HIP_PREFILL_DIGITS");
     const bool attn_digits = !(digits_env != nullptr && digits_env[0] == '0');
-    if (out != hidden_in &&
-        hipMemcpyAsync(out, hidden_in, batch * hidden * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess) {
-        return TE_STATUS_RUNTIME_ERROR;
-    }
     const size_t ctx_kv = context_tokens * kv;
     const size_t vt_layer = te_hip_value_t_bytes(1, 1, context_tokens, kv_heads, head_dim) / sizeof(uint16_t);
     te_hip::prof_begin(st);
@@ -261,7 +257,7 @@ static te_status prefill_all_layers_impl(
         // the attention RMSNorm operand of layer l > 0 came with the previous
         // layer's down projection
         if ((l == 0 && !done((stage_name = "attn_norm_digits",
-                              s = te_hip::launch_split_act(1, out, nullptr, attn_norm_weights, epsilon, batch, hidden,
+                              s = te_hip::launch_split_act(1, hidden_in, nullptr, attn_norm_weights, epsilon, batch, hidden,
                                                            b.act, st)),
                              ew)) ||
             !qkv_done((stage_name = "qkv_proj",
@@ -283,7 +279,7 @@ static te_status prefill_all_layers_impl(
                    ew)) ||
             !done((stage_name = "output_proj_add_ffn_norm_digits",
                    s = te_hip::launch_gemm_q_rms(m + output_offsets[l], ggml_type, b.act, batch, hidden, hidden, out,
-                                                 out, b.part, b.part_bytes, ffn_norm_weights + l * hidden, epsilon,
+                                                 l == 0 ? hidden_in : out, b.part, b.part_bytes, ffn_norm_weights + l * hidden, epsilon,
                                                  b.act, st)),
                   te_hip::kProfO) ||
             !glu_done(s = te_hip::launch_gemm_glu_q(ggml_type, m + gate_offsets[l], m + up_offsets[l], b.act, batch,

@@ -572,7 +572,8 @@ __device__ __forceinline__ float pair_dot(const uint32_t *w, const uint32_t (&xq
 template <uint32_t TYPE, int LPR, int NR>
 __global__ __launch_bounds__(kPairThreads) void matvec_pairs_kernel(const unsigned char *weights,
                                                                        const float *input, int cols, int rows,
-                                                                       size_t row_bytes, float *out, int tiles) {
+                                                                       size_t row_bytes, float *out,
+                                                                       const float *resid, int tiles) {
     constexpr int PW = TYPE == kGgmlQ4_0 ? 9 : 17;  // dwords per block pair
     constexpr int G = 64 / LPR;                      // row groups per wave
     extern __shared__ uint4 xs_lds4[];  // [pairs][13] uint4: block 0 planes, block 1 planes, scales
@@ -664,7 +665,7 @@ __global__ __launch_bounds__(kPairThreads) void matvec_pairs_kernel(const unsign
             }
             const int row = (tile * G + grp) * NR + r;
             if (li == 0 && row < rows) {
-                out[row] = v;
+                out[row] = resid != nullptr ? resid[row] + v : v;
             }
             acc[r] = 0.0f;
         }
@@ -1249,13 +1250,18 @@ te_status launch_stream(uint32_t ggml_type, int pre, StreamArgs a, hipStream_t s
     return launch_status();
 }
 
+// Whether launch_matvec adds a residual itself (every launch but F32 rows and odd block counts).
+static bool matvec_adds(uint32_t ggml_type, size_t cols) {
+    return ggml_type != kGgmlF32 && cols % 64 == 0 && cols / 64 * kPairLdsBytes <= kMaxPairLdsBytes;
+}
+
 te_status launch_matvec(const void *weights, uint32_t ggml_type, const float *input, size_t cols, size_t rows,
-                        float *out, hipStream_t stream) {
+                        float *out, hipStream_t stream, const float *resid) {
     const size_t row_bytes = ggml_row_bytes(ggml_type, cols);
     const unsigned char *w = static_cast<const unsigned char *>(weights);
     const size_t waves_wanted = (size_t)device_compute_units() * 16;
     const size_t pair_lds_bytes = cols / 64 * kPairLdsBytes;
-    if (ggml_type != kGgmlF32 && cols % 64 == 0 && pair_lds_bytes <= kMaxPairLdsBytes) {
+    if (matvec_adds(ggml_type, cols)) {
         // block pairs: lanes per row from the pair count; rows per group so that the
         // tiles give every CU at least 8 waves where the rows allow (Q8_0 stays at two
         // rows: four double-buffered 68-byte pairs do not fit 3 waves per SIMD)
@@ -1266,7 +1272,7 @@ te_status launch_matvec(const void *weights, uint32_t ggml_type, const float *in
         const size_t want = cus * 8;
         if (getenv("TE_HIP_GEMV_STRIDED") == nullptr) {
             StreamArgs a = {};
-            a.seg[0] = StreamSeg{w, out, nullptr, 0, (int)rows, 0};
+            a.seg[0] = StreamSeg{w, out, resid, 0, (int)rows, 0};
             a.nseg = 1;
             a.cols = (int)cols;
             a.in = StageInput{input, nullptr, nullptr, 0.0f};
@@ -1292,7 +1298,7 @@ te_status launch_matvec(const void *weights, uint32_t ggml_type, const float *in
             return TE_STATUS_RUNTIME_ERROR;                                                                       \
         }                                                                                                         \
         matvec_pairs_kernel<T, L, N><<<grid, block, pair_lds_bytes, stream>>>(w, input, (int)cols, (int)rows,     \
-                                                                             row_bytes, out, (int)tiles);         \
+                                                                             row_bytes, out, resid, (int)tiles);         \
     } while (0)
 #define TE_PAIRS_NR(T, L)                                    \
     do {                                                     \
@@ -1381,8 +1387,10 @@ te_status launch_gemv(uint32_t ggml_type, GemvPre pre, const GemvSeg *segs, int 
         input = xtmp;
     }
     for (int s = 0; s < nseg && st == TE_STATUS_OK; ++s) {
-        if (segs[s].resid == nullptr) {
-            st = launch_matvec(segs[s].w, ggml_type, input, cols, segs[s].rows, segs[s].out, stream);
+        // rows past the streamed kernel's tile (7B Q8_0 ffn_down, 20 KB) add
+        // the residual as they are stored: an add launch took 4.1 us
+        if (segs[s].resid == nullptr || matvec_adds(ggml_type, cols)) {
+            st = launch_matvec(segs[s].w, ggml_type, input, cols, segs[s].rows, segs[s].out, stream, segs[s].resid);
         } else {
             st = launch_matvec(segs[s].w, ggml_type, input, cols, segs[s].rows, ytmp, stream);
             if (st == TE_STATUS_OK) {
