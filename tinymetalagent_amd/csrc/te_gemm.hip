@@ -98,6 +98,14 @@ __device__ __forceinline__ double row_sum_squares(double ss) {
     return t;
 }
 
+// Row of workgroup id: workgroups go to the XCDs round-robin, and eight
+// consecutive rows share each 128-byte line of the operand, so an XCD takes
+// consecutive rows.
+__host__ __device__ inline size_t xcd_rows(size_t rows) { return (rows + 63) / 64 * 8; }  // per XCD
+__device__ __forceinline__ size_t xcd_row(unsigned id, int rows) {
+    return (id & 7) * xcd_rows((size_t)rows) + (id >> 3);
+}
+
 // x' = pre(x) as the GEMM's hi / lo operand.  Thread t of a workgroup holds
 // eight consecutive values of block t / 4 of a pass of 64 blocks; without a
 // row-wide norm the gridDim.y workgroups of a row take every gridDim.y-th
@@ -109,8 +117,11 @@ template <int PRE>
 __global__ __launch_bounds__(kActThreads) void split_act_kernel(const float *__restrict__ x,
                                                                 const float *__restrict__ x2,
                                                                 const float *__restrict__ norm_w, float eps,
-                                                                int K, unsigned char *__restrict__ act, bool vec) {
-    const size_t row = blockIdx.x;
+                                                                int M, int K, unsigned char *__restrict__ act, bool vec) {
+    const size_t row = xcd_row(blockIdx.x, M);
+    if (row >= (size_t)M) {
+        return;
+    }
     const float *xr = x + row * (size_t)K;
     const int c0 = 8 * (int)threadIdx.x;
     float rms = 1.0f;
@@ -606,10 +617,13 @@ __global__ __launch_bounds__(256) void gemm_reduce_segs_kernel(const float *__re
 constexpr int kRmsSplits = 16;  // also the most splits of a launch
 __global__ __launch_bounds__(kActThreads) void gemm_reduce_rms_kernel(const float *__restrict__ part, int splits,
                                                                       size_t count, const float *resid, float *out,
-                                                                      int N, const float *__restrict__ norm_w,
+                                                                      int M, int N, const float *__restrict__ norm_w,
                                                                       float eps, unsigned char *__restrict__ act,
                                                                       bool vec) {
-    const size_t row = blockIdx.x;
+    const size_t row = xcd_row(blockIdx.x, M);
+    if (row >= (size_t)M) {
+        return;
+    }
     const int c = 8 * (int)threadIdx.x;
     const bool mine = c < N;
     const int cl = mine ? c : 0;  // threads past the row load column 0 and store nothing
@@ -691,13 +705,13 @@ te_status launch_split_act(int pre, const float *x, const float *x2, const float
     unsigned char *a = act_base(act);
     const bool vec = aligned16(x) && (pre != kActSwiGLU || aligned16(x2)) && (pre != kActRmsNorm || aligned16(norm_w));
     // without a row-wide norm, the row's passes of kActPass values are spread over workgroups
-    const dim3 grid((unsigned)rows, pre == kActRmsNorm ? 1u : (unsigned)std::max<size_t>(1, cols / kActPass));
+    const dim3 grid((unsigned)(8 * xcd_rows(rows)), pre == kActRmsNorm ? 1u : (unsigned)std::max<size_t>(1, cols / kActPass));
     if (pre == kActRmsNorm) {
-        split_act_kernel<kActRmsNorm><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, a, vec);
+        split_act_kernel<kActRmsNorm><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)rows, (int)cols, a, vec);
     } else if (pre == kActSwiGLU) {
-        split_act_kernel<kActSwiGLU><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, a, vec);
+        split_act_kernel<kActSwiGLU><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)rows, (int)cols, a, vec);
     } else {
-        split_act_kernel<kActPlain><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)cols, a, vec);
+        split_act_kernel<kActPlain><<<grid, kActThreads, 0, stream>>>(x, x2, norm_w, eps, (int)rows, (int)cols, a, vec);
     }
     return launch_status();
 }
@@ -862,8 +876,8 @@ te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, 
         const unsigned blocks = (unsigned)std::min<size_t>((count / width + 255) / 256, 4096);
         const char *env = getenv("TE_HIP_GEMM_REDUCE_RMS");
         if (rms && n <= (size_t)kActPass && splits <= (size_t)kRmsSplits && !(env != nullptr && env[0] == '0')) {
-            gemm_reduce_rms_kernel<<<(unsigned)rows, kActThreads, 0, stream>>>(
-                partials, (int)splits, count, res, out, (int)n, post->norm_w, post->eps, act_base(post->act_out),
+            gemm_reduce_rms_kernel<<<(unsigned)(8 * xcd_rows(rows)), kActThreads, 0, stream>>>(
+                partials, (int)splits, count, res, out, (int)rows, (int)n, post->norm_w, post->eps, act_base(post->act_out),
                 vec && aligned16(post->norm_w));
             rms_done = true;
         } else if (nseg == 1) {
