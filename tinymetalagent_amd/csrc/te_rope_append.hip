@@ -229,14 +229,17 @@ struct KvAppendVtArgs {
     int kv_heads;
 };
 
-template <int D>
+// PREFIX: V^T of the cached positions before the chunk as well (0 .. base - 1,
+// read from the value cache), for a caller that keeps no V^T.
+template <int D, bool PREFIX>
 __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
     constexpr int P = 32;  // positions per workgroup (64 measured 5 % slower at 512 tokens)
     constexpr int HALF = D / 2;
     __shared__ __attribute__((aligned(16))) f16 tile[P][D + 8];
     const int first = a.base;
     const int end = a.base + a.tokens;
-    const int p0 = (first & ~(P - 1)) + P * (int)blockIdx.x;
+    const int vt_first = PREFIX ? 0 : first;
+    const int p0 = (vt_first & ~(P - 1)) + P * (int)blockIdx.x;
     const int h = blockIdx.y;
     const int sl = blockIdx.z;
     const int layer = sl % a.layers;
@@ -254,8 +257,10 @@ __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
     static_assert(KI * 256 == P * (HALF / 4) && VI * 256 == P * (D / 8), "items tile the workgroup");
     float4 k0[KI], k1[KI], c4[KI], s4[KI], kb0[KI], kb1[KI];
     float4 v0[VI], v1[VI], vb0[VI], vb1[VI];
+    f16x8 vc[VI];
+    const bool chunk = !PREFIX || p0 + P > first;  // some position of the chunk (uniform)
 #pragma unroll
-    for (int u = 0; u < KI; ++u) {
+    for (int u = 0; chunk && u < KI; ++u) {
         const int idx = threadIdx.x + 256 * u;
         const int r = idx / (HALF / 4);
         const int i = 4 * (idx % (HALF / 4));
@@ -279,6 +284,11 @@ __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
         const int p = p0 + r;
         const int pl = p >= first && p < end ? p : first;
         const float *vrow = a.v + ((size_t)sl * a.tokens + (pl - first)) * kv_dim + h * D + 8 * cq;
+        if (PREFIX && p < first) {
+            vc[u] = *reinterpret_cast<const f16x8 *>(a.value_cache + ((size_t)sl * a.ctx + p) * kv_dim + h * D +
+                                                     8 * cq);
+            continue;
+        }
         v0[u] = *reinterpret_cast<const float4 *>(vrow);
         v1[u] = *reinterpret_cast<const float4 *>(vrow + 4);
         if (vb != nullptr) {
@@ -288,7 +298,7 @@ __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
     }
     // k: bias, rotation, fp16 (rope_kv_append_kernel's operation order)
 #pragma unroll
-    for (int u = 0; u < KI; ++u) {
+    for (int u = 0; chunk && u < KI; ++u) {
         const int idx = threadIdx.x + 256 * u;
         const int r = idx / (HALF / 4);
         const int i = 4 * (idx % (HALF / 4));
@@ -327,7 +337,9 @@ __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
         const int cq = idx % (D / 8);
         const int p = p0 + r;
         f16x8 val = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (p >= first && p < end) {
+        if (PREFIX && p < first) {
+            val = vc[u];
+        } else if (p >= first && p < end) {
             float x[8] = {v0[u].x, v0[u].y, v0[u].z, v0[u].w, v1[u].x, v1[u].y, v1[u].z, v1[u].w};
             if (vb != nullptr) {
                 const float b[8] = {vb0[u].x, vb0[u].y, vb0[u].z, vb0[u].w, vb1[u].x, vb1[u].y, vb1[u].z, vb1[u].w};
@@ -350,7 +362,7 @@ __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
         const int i = idx / (P / 8);
         const int pc = idx % (P / 8);
         const int pa = p0 + 8 * pc;
-        if (pa >= a.end8 || pa + 8 <= first) {
+        if (pa >= a.end8 || pa + 8 <= vt_first) {
             continue;
         }
         f16x8 val;
@@ -359,12 +371,12 @@ __global__ __launch_bounds__(256) void kv_append_vt_kernel(KvAppendVtArgs a) {
             val[j] = tile[8 * pc + j][i];
         }
         f16 *row = dst + (size_t)i * a.ctx_pad + pa;
-        if (pa >= first && pa + 8 <= a.end8) {
+        if (pa >= vt_first && pa + 8 <= a.end8) {
             *reinterpret_cast<f16x8 *>(row) = val;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                if (pa + j >= first && pa + j < a.end8) {
+                if (pa + j >= vt_first && pa + j < a.end8) {
                     row[j] = val[j];
                 }
             }
@@ -426,7 +438,7 @@ te_status launch_kv_append_vt(const float *k, const float *v, const float *k_bia
                               const float *rope_cos, const float *rope_sin, uint16_t *key_cache,
                               uint16_t *value_cache, uint16_t *value_t, size_t sl_count, size_t layers,
                               size_t tokens, size_t base_position, size_t context_tokens, size_t ctx_pad,
-                              size_t kv_heads, size_t head_dim, hipStream_t stream) {
+                              size_t kv_heads, size_t head_dim, bool prefix, hipStream_t stream) {
     if ((head_dim != 64 && head_dim != 128) || tokens == 0 || ctx_pad < base_position + tokens ||
         ctx_pad % 64 != 0 || sl_count > 65535 || kv_heads > 65535) {
         return TE_STATUS_INVALID_ARGUMENT;
@@ -449,12 +461,19 @@ te_status launch_kv_append_vt(const float *k, const float *v, const float *k_bia
     a.ctx = (int)context_tokens;
     a.ctx_pad = (int)ctx_pad;
     a.kv_heads = (int)kv_heads;
-    const size_t tiles = ((size_t)a.end8 - (base_position & ~(size_t)31) + 31) / 32;
+    prefix = prefix && base_position > 0;
+    const size_t tiles = ((size_t)a.end8 - (prefix ? 0 : base_position & ~(size_t)31) + 31) / 32;
     const dim3 grid((unsigned)tiles, (unsigned)kv_heads, (unsigned)sl_count);
     if (head_dim == 128) {
-        kv_append_vt_kernel<128><<<grid, 256, 0, stream>>>(a);
+        if (prefix) {
+            kv_append_vt_kernel<128, true><<<grid, 256, 0, stream>>>(a);
+        } else {
+            kv_append_vt_kernel<128, false><<<grid, 256, 0, stream>>>(a);
+        }
+    } else if (prefix) {
+        kv_append_vt_kernel<64, true><<<grid, 256, 0, stream>>>(a);
     } else {
-        kv_append_vt_kernel<64><<<grid, 256, 0, stream>>>(a);
+        kv_append_vt_kernel<64, false><<<grid, 256, 0, stream>>>(a);
     }
     return launch_status();
 }
