@@ -45,9 +45,9 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 METRIC = "decode-attn µs/layer + HBM GB/s (% peak) at Qwen2.5-3B, ctx 8K; prefill TFLOP/s"
-INT8_MFMA_PEAK_TOPS = 5000.0  # MI355X dense int8 MFMA, TOP/s
 HBM_PEAK_GBS = 8000.0
 FP16_MFMA_PEAK_TFLOPS = 2500.0
+BF16_MFMA_PEAK_TFLOPS = 2500.0
 THETA = 1e6
 
 
@@ -727,11 +727,11 @@ def decode_layers_case(torch, LY, V, ggml_type: int, *, layers=36, heads=16, kv_
 
 
 def gemm_case(torch, ggml_type: int, rows: int, n: int, k: int, pre: int = 0, reps: int = 20) -> dict:
-    """te_hip_gemm_q_f32 (the batched-prefill projection: activation digits +
-    int8-MFMA GEMM) at one prompt-chunk shape, graph-replayed over weight
-    copies rotated past the MALL.  Algorithmic work: rows * n * k multiply-adds,
-    priced against the dense int8 MFMA peak at two int8 products per
-    multiply-add (two activation digits) and, as `frac_algorithmic`, at one."""
+    """te_hip_gemm_q_f32 (the batched-prefill projection: activations as bf16
+    hi + lo + a bf16-MFMA GEMM) at one prompt-chunk shape, graph-replayed over
+    weight copies rotated past the MALL.  Algorithmic work: rows * n * k
+    multiply-adds, priced against the dense bf16 MFMA peak at two bf16 products
+    per multiply-add (hi and lo) and, as `frac_algorithmic`, at one."""
     from tinymetalagent_amd import runtime as R
     lib = R.load_library()
     rb = k // 32 * (18 if ggml_type == 2 else 34)
@@ -758,8 +758,8 @@ def gemm_case(torch, ggml_type: int, rows: int, n: int, k: int, pre: int = 0, re
     del ws
     torch.cuda.empty_cache()
     return {"rows": rows, "n": n, "k": k, "us": r(us, 2), "algorithmic_tops": round(tops, 1),
-            "int8_mfma_tops": round(2 * tops, 1), "frac": r(2 * tops / INT8_MFMA_PEAK_TOPS),
-            "frac_algorithmic": r(tops / INT8_MFMA_PEAK_TOPS)}
+            "bf16_mfma_tflops": round(2 * tops, 1), "frac": r(2 * tops / BF16_MFMA_PEAK_TFLOPS),
+            "frac_algorithmic": r(tops / BF16_MFMA_PEAK_TFLOPS)}
 
 
 def write_3b_gguf(path: str, ggml_type: int, *, layers=36, heads=16, kv_heads=2, d=128, ffn=11008,
@@ -824,7 +824,7 @@ def write_3b_gguf(path: str, ggml_type: int, *, layers=36, heads=16, kv_heads=2,
 def generate_case(ggml_type: int, prompt_tokens: int = 512, new_tokens: int = 128, ctx: int = 1024) -> dict:
     """End-to-end te_generate_raw on a 3B-shaped GGUF through the public C ABI
     (the reference's own entry point, qwen.c:261-400): load, a prompt of
-    `prompt_tokens` byte tokens through the batched prefill (int8-MFMA prompt
+    `prompt_tokens` byte tokens through the batched prefill (bf16-MFMA prompt
     GEMMs and causal attention over 512-row chunks,
     te_hip_prefill_all_layers_f16), then greedy decode with every token
     streamed to the callback.  Times: load (parse + upload of
@@ -1237,7 +1237,7 @@ def main():
         # generation through the public C ABI on a 3B-shaped GGUF
         line["generate"] = {
             "workload": "te_generate_raw on a Qwen2.5-3B-shaped GGUF (random weights, 151936-token byte-level "
-                        "vocabulary): 512 prompt tokens through the batched int8-MFMA prefill (512-row chunks), "
+                        "vocabulary): 512 prompt tokens through the batched bf16-MFMA prefill (512-row chunks), "
                         "then 128 greedy tokens; ctx 1024",
             "q4_0": generate_case(2),
             "prefill_gemm_gate_q4_0": gemm_case(torch, 2, 512, 11008, 2048, pre=1),

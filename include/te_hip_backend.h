@@ -112,7 +112,9 @@ TE_API te_status te_hip_rope_kv_append_f16(
  * on demand, guarded by the library mutex; calls using it must all go to one
  * stream).  Calls sharing one workspace must be stream-ordered.  The chunking
  * depends on all positions, not only the longest (the chunk length balances
- * the total work over the GPU's wave slots); the workspace size depends only
+ * the total work over the GPU's wave slots, and a sequence's chunks are equal
+ * in length, so a shorter sequence of a batch can have shorter ones); the
+ * workspace size depends only
  * on the largest position and never decreases with it.
  */
 TE_API size_t te_hip_attention_decode_workspace_bytes(const size_t *positions, size_t position, size_t seqs,
@@ -121,7 +123,7 @@ TE_API size_t te_hip_attention_decode_workspace_bytes(const size_t *positions, s
 
 /*
  * The chunking behind the decode entry points: *chunk = cache positions per
- * split-K workgroup, *chunks = chunks of the longest sequence.  fp32_cache != 0
+ * split-K workgroup (the most of any sequence), *chunks = chunks of the longest sequence.  fp32_cache != 0
  * gives the chunking of te_attention_decode_f32 (seqs == layers == 1; a
  * power-of-two multiple of 512 positions, at most 4096 chunks for any
  * position).  A host computation from the sizes and the device's compute-unit
@@ -202,8 +204,9 @@ TE_API te_status te_hip_attention_decode_step_splitk_f16(
  * (16 MiB) per GPU, held from first use until the process ends.  The call
  * allocates nothing.  A call whose partials
  * (seqs*layers*heads*chunks*(head_dim+2)*4 bytes, chunks as reported by
- * te_hip_attention_decode_chunking) exceed the array returns
- * TE_STATUS_UNSUPPORTED before any work is queued.  Every call on one GPU
+ * te_hip_attention_decode_chunking) exceed the array takes the longer chunks
+ * that fit it; one that fits with none returns TE_STATUS_UNSUPPORTED before
+ * any work is queued.  Every call on one GPU
  * shares the array: calls that overlap in time on one GPU (different streams,
  * different threads) race and must be ordered by the caller.
  */
