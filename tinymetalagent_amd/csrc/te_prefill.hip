@@ -822,33 +822,12 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_causal_f16_kernel(Prefill
                 // dims 16t + 4g + r of the lane's row
                 *reinterpret_cast<f32x4 *>(stg + c * OPITCH + 16 * t + 4 * g) = ob[t] * w1 + po[t] * w2;
             }
+            constexpr int LPR = D / 4;          // lanes per row: 16 bytes each
+            constexpr int NS = 16 * LPR / 64;   // rows per lane
             // (the lane index is opaque here, so the row addresses are formed
             // here rather than kept live across the step loop)
             int ln = lane;
             asm volatile("" : "+v"(ln));
-            const int row0 = wr0 + 16 * nb;
-            if constexpr (MODE == kQ32Act) {
-                // the operand holds 16 bytes of a row's eight columns beside the
-                // next row's: two lanes a piece, all 16 rows of two column groups
-                // an instruction (256 contiguous bytes a group; by rows, in pieces
-                // of 32 bytes, 7B 512 rows took 26.4 us against 24.9)
-                const int r = (ln >> 1) & 15;
-                const int q = 8 * (ln >> 5) + 4 * (ln & 1);
-                f32x4 v[D / 16];
-#pragma unroll
-                for (int i = 0; i < D / 16; ++i) {
-                    v[i] = *reinterpret_cast<const f32x4 *>(stg + r * OPITCH + 16 * i + q);
-                }
-                if (row0 + r < a.tokens) {
-#pragma unroll
-                    for (int i = 0; i < D / 16; ++i) {
-                        store_act4(v[i], (size_t)sl * a.tokens + row0 + r, a.heads * D, h * D + 16 * i + q, a.act);
-                    }
-                }
-                return;
-            }
-            constexpr int LPR = D / 4;          // lanes per row: 16 bytes each
-            constexpr int NS = 16 * LPR / 64;   // rows per lane
             const int r0 = (int)((unsigned)ln / LPR);
             const int q = (int)((unsigned)ln % LPR);
             // every staged piece is read before the first store, so the stores
@@ -861,6 +840,17 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_causal_f16_kernel(Prefill
             // rows row0 + r, r = i * (64 / LPR) + r0, of this (seq*layer, head):
             // a 32-bit float offset from the block's first row (16 rows of
             // heads * D floats)
+            const int row0 = wr0 + 16 * nb;
+            if constexpr (MODE == kQ32Act) {
+#pragma unroll
+                for (int i = 0; i < NS; ++i) {
+                    const int r = i * (64 / LPR) + r0;
+                    if (row0 + r < a.tokens) {
+                        store_act4(v[i], (size_t)sl * a.tokens + row0 + r, a.heads * D, h * D + 4 * q, a.act);
+                    }
+                }
+                return;
+            }
             float *orow = a.out + (((size_t)sl * a.tokens + row0) * a.heads + h) * D;
             const unsigned rstride = (unsigned)a.heads * D;
             // non-temporal: the output is not read back by this launch
@@ -1231,39 +1221,25 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_rows_f16_kernel(PrefillAr
 #ifdef TE_PREFILL_PHASES
     tr[4] = (unsigned)__builtin_amdgcn_s_memrealtime();
 #endif
-    if (a.act != nullptr) {  // uniform
-        // wave w: column groups w, w + 8 of all 32 rows: the operand holds a
-        // row's eight columns beside the next row's, so a group leaves as 512
-        // contiguous bytes (by rows, in pieces of 32 bytes, 3B 512 rows took
-        // 18.0 us against 16.8)
-        const int r = (lane >> 1) & 31;
+    // wave w: rows 4w .. 4w + 3 of the group, LPR lanes of 16 bytes per row
+    constexpr int LPR = D / 4;
+    constexpr int RPP = 64 / LPR;  // rows per pass
+    const int q = lane % LPR;
 #pragma unroll
-        for (int i = 0; i < D / 64; ++i) {
-            const int col = 8 * (wave + 8 * i) + 4 * (lane & 1);
-            f32x4 acc = *reinterpret_cast<const f32x4 *>(&part[0][r * OPITCH + col]);
-            for (int p = 1; p < nact; ++p) {
-                acc += *reinterpret_cast<const f32x4 *>(&part[p][r * OPITCH + col]);
-            }
-            if (r0 + r < a.tokens) {
-                store_act4(acc, (size_t)sl * a.tokens + r0 + r, a.heads * D, h * D + col, a.act);
-            }
+    for (int i = 0; i < 4 / RPP; ++i) {
+        const int r = 4 * wave + i * RPP + lane / LPR;
+        f32x4 acc = *reinterpret_cast<const f32x4 *>(&part[0][r * OPITCH + 4 * q]);
+        for (int p = 1; p < nact; ++p) {
+            acc += *reinterpret_cast<const f32x4 *>(&part[p][r * OPITCH + 4 * q]);
         }
-    } else {
-        // wave w: rows 4w .. 4w + 3 of the group, LPR lanes of 16 bytes per row
-        constexpr int LPR = D / 4;
-        constexpr int RPP = 64 / LPR;  // rows per pass
-        const int q = lane % LPR;
-#pragma unroll
-        for (int i = 0; i < 4 / RPP; ++i) {
-            const int r = 4 * wave + i * RPP + lane / LPR;
-            f32x4 acc = *reinterpret_cast<const f32x4 *>(&part[0][r * OPITCH + 4 * q]);
-            for (int p = 1; p < nact; ++p) {
-                acc += *reinterpret_cast<const f32x4 *>(&part[p][r * OPITCH + 4 * q]);
-            }
-            if (r0 + r < a.tokens) {
-                float *orow = a.out + (((size_t)sl * a.tokens + r0 + r) * a.heads + h) * D;
-                __builtin_nontemporal_store(acc, reinterpret_cast<f32x4 *>(orow + 4 * q));
-            }
+        if (r0 + r >= a.tokens) {
+            continue;
+        }
+        if (a.act != nullptr) {  // uniform
+            store_act4(acc, (size_t)sl * a.tokens + r0 + r, a.heads * D, h * D + 4 * q, a.act);
+        } else {
+            float *orow = a.out + (((size_t)sl * a.tokens + r0 + r) * a.heads + h) * D;
+            __builtin_nontemporal_store(acc, reinterpret_cast<f32x4 *>(orow + 4 * q));
         }
     }
 #ifdef TE_PREFILL_PHASES
