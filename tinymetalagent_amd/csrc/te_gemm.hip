@@ -610,61 +610,84 @@ __global__ __launch_bounds__(256) void gemm_reduce_segs_kernel(const float *__re
 // gemm_reduce_kernel's sums for one row (resid + the splits' partial sums in
 // split order -> out), then that row's RMSNorm operand into act, exactly as
 // split_act_kernel<kActRmsNorm> computes it from out: thread t holds columns
-// 8t .. 8t + 7, summed into the fp64 sum of squares in row_sum_squares's order,
-// and splits them as split_act_kernel's thread t does.  One workgroup per row, N <= kActPass, N % 32 == 0,
-// splits <= kRmsSplits.  Every load, the norm weights' included, is issued
-// before the first store (out may be resid), so all of a thread's loads are
-// in flight together.
+// 8t .. 8t + 7 of each of P passes of kActPass, summed into the fp64 sum of
+// squares in row_sum_squares's order, and splits them as split_act_kernel's
+// thread t does.  One workgroup per row, N <= P * kActPass, N % 32 == 0,
+// splits <= rms_splits(P) (what the registers hold).  Every load, the norm weights' included, is issued before the
+// first store (out may be resid), so all of a thread's loads are in flight
+// together.  Bound by its two rounds of latency (loads, the row's sum) and the
+// launch; two passes of 256 threads rather than 512 threads keep
+// split_act_kernel's sum order.  P = 2 against the separate sums and operand
+// launches, 7B, two layers (three such places): Q4_0 181 rows 613.9 -> 610.3
+// us, 12 rows 321.5 -> 319.4, Q8_0 21 rows 395.2 -> 392.4.
 constexpr int kRmsSplits = 16;  // also the most splits of a launch
+// (P = 2: 228 VGPRs, two waves per SIMD; a 7B down takes up to 9 splits)
+constexpr int rms_splits(int passes) { return passes == 1 ? kRmsSplits : 12; }
+template <int P>
 __global__ __launch_bounds__(kActThreads) void gemm_reduce_rms_kernel(const float *__restrict__ part, int splits,
                                                                       size_t count, const float *resid, float *out,
                                                                       int M, int N, const float *__restrict__ norm_w,
                                                                       float eps, unsigned char *__restrict__ act,
                                                                       bool vec) {
+    constexpr int S = rms_splits(P);
     const size_t row = xcd_row(blockIdx.x, M);
     if (row >= (size_t)M) {
         return;
     }
-    const int c = 8 * (int)threadIdx.x;
-    const bool mine = c < N;
-    const int cl = mine ? c : 0;  // threads past the row load column 0 and store nothing
-    const size_t o = row * (size_t)N + cl;
-    float pv[kRmsSplits][8], rv[8] = {}, wv[8];
+    const int c0 = 8 * (int)threadIdx.x;
+    const size_t o0 = row * (size_t)N;
+    float pv[P][S][8], rv[P][8] = {}, wv[P][8];
 #pragma unroll
-    for (int z = 0; z < kRmsSplits; ++z) {
-        if (z < splits) {
-            load8(part + (size_t)z * count + o, vec, pv[z]);
-        }
-    }
-    if (resid != nullptr) {
-        load8(resid + o, vec, rv);
-    }
-    load8(norm_w + cl, vec, wv);
-    float xv[8];
-    double ss = 0.0;
+    for (int i = 0; i < P; ++i) {
+        const int c = c0 + i * kActPass;
+        const int cl = c < N ? c : 0;  // threads past the row load column 0 and store nothing
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        float a = pv[0][j];
-#pragma unroll
-        for (int z = 1; z < kRmsSplits; ++z) {
+        for (int z = 0; z < S; ++z) {
             if (z < splits) {
-                a += pv[z][j];
+                load8(part + (size_t)z * count + o0 + cl, vec, pv[i][z]);
             }
         }
-        xv[j] = resid != nullptr ? rv[j] + a : a;
-        const double d = (double)xv[j];
-        ss += mine ? d * d : 0.0;
+        if (resid != nullptr) {
+            load8(resid + o0 + cl, vec, rv[i]);
+        }
+        load8(norm_w + cl, vec, wv[i]);
     }
-    if (mine) {
-        store8(out + o, vec, xv);
-    }
-    const float rms = 1.0f / sqrtf((float)(row_sum_squares(ss) / (double)N) + eps);
-    if (mine) {
+    float xv[P][8];
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const bool mine = c0 + i * kActPass < N;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            xv[j] = xv[j] * rms * wv[j];
+            float a = pv[i][0][j];
+#pragma unroll
+            for (int z = 1; z < S; ++z) {
+                if (z < splits) {
+                    a += pv[i][z][j];
+                }
+            }
+            xv[i][j] = resid != nullptr ? rv[i][j] + a : a;
+            const double d = (double)xv[i][j];
+            ss += mine ? d * d : 0.0;
         }
-        split_store8(xv, row, N >> 5, c, act);
+    }
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        if (c0 + i * kActPass < N) {
+            store8(out + o0 + c0 + i * kActPass, vec, xv[i]);
+        }
+    }
+    const float rms = 1.0f / sqrtf((float)(row_sum_squares(ss) / (double)N) + eps);
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int c = c0 + i * kActPass;
+        if (c < N) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                xv[i][j] = xv[i][j] * rms * wv[i][j];
+            }
+            split_store8(xv[i], row, N >> 5, c, act);
+        }
     }
 }
 
@@ -876,8 +899,12 @@ te_status launch_gemm_q_segs(uint32_t ggml_type, const GemmSeg *segs, int nseg, 
         const int width = vec ? 4 : 1;
         const unsigned blocks = (unsigned)std::min<size_t>((count / width + 255) / 256, 4096);
         const char *env = getenv("TE_HIP_GEMM_REDUCE_RMS");
-        if (rms && n <= (size_t)kActPass && splits <= (size_t)kRmsSplits && !(env != nullptr && env[0] == '0')) {
-            gemm_reduce_rms_kernel<<<(unsigned)(8 * xcd_rows(rows)), kActThreads, 0, stream>>>(
+        // one pass of a row up to 2048 wide, two up to 4096 (the 7B width); wider
+        // rows take two launches, as the registers hold no third pass
+        const size_t passes = (n + kActPass - 1) / kActPass;
+        if (rms && passes <= 2 && splits <= (size_t)rms_splits((int)passes) && !(env != nullptr && env[0] == '0')) {
+            auto *kernel = passes == 1 ? gemm_reduce_rms_kernel<1> : gemm_reduce_rms_kernel<2>;
+            kernel<<<(unsigned)(8 * xcd_rows(rows)), kActThreads, 0, stream>>>(
                 partials, (int)splits, count, res, out, (int)rows, (int)n, post->norm_w, post->eps, act_base(post->act_out),
                 vec && aligned16(post->norm_w));
             rms_done = true;
