@@ -1,5 +1,7 @@
 """The fused decode step over batches of ragged sequences, whose chunks are
-numbered one after another over the sequences: every sequence of the batch
+numbered one after another over the sequences (chunks first, or the streams of
+a layer and KV head first where there are few long chunks; the longest cut
+finer where the lengths differ): every sequence of the batch
 against the same step run on it alone (the same arithmetic over another cut of
 its positions), the appended rows bit for bit, and the array-backed entry
 point, which cuts a batch no finer than its array holds.
@@ -31,7 +33,11 @@ def _inputs(seqs, layers, ctx, heads, kv, d):
 
 @pytest.mark.parametrize("layers,heads,kv,d,positions", [
     (1, 14, 2, 64, [0, 31]), (3, 8, 2, 128, [32, 0, 511, 63, 64, 1000]), (2, 4, 1, 64, [700] * 8),
-    (1, 2, 2, 128, [(37 * i) % 650 for i in range(64)]), (40, 16, 2, 128, [5, 3000, 255, 256, 257])])
+    (1, 2, 2, 128, [(37 * i) % 650 for i in range(64)]), (40, 16, 2, 128, [5, 3000, 255, 256, 257]),
+    # streams first: one chunk each, and up to three
+    (28, 8, 4, 64, [600, 598, 601, 599, 577, 575, 576, 300, 600, 544]), (28, 8, 4, 128, [1500, 900, 1503, 1501, 31]),
+    # cut finer: 8 chunks of the longest
+    (28, 8, 4, 64, [2000, 10, 20, 300, 50, 40, 60, 100])])
 def test_ragged_batch_matches_each_sequence_alone(layers, heads, kv, d, positions):
     ctx = max(positions) + 1
     q, k, v, cos, sin, kc, vc = _inputs(len(positions), layers, ctx, heads, kv, d)

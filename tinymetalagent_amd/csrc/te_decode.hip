@@ -75,11 +75,12 @@ struct DecodeArgs {
     int kv_heads;
     int group;
     int seqs;
+    int streams_first;  // grid (KV head, layer, chunk) instead of (chunk, KV head, layer)
     int max_chunks;
     float qscale;    // log2(e)/sqrt(D)
     int positions[TE_HIP_MAX_SEQS];
-    // sequence s has chunks first[s] .. first[s + 1] - 1 of the launch's list
-    // (grid.x), of ceil(tiles / chunks) tiles each
+    // sequence s has chunks first[s] .. first[s + 1] - 1 of the launch's list,
+    // of ceil(tiles / chunks) tiles each
     int first[TE_HIP_MAX_SEQS + 1];
 };
 
@@ -281,15 +282,17 @@ __global__ __launch_bounds__(64, 2) void decode_splitk_f16_kernel(DecodeArgs a) 
     constexpr int KK = D / 32;  // MFMA K-steps over head_dim for QK^T
 
     const int lane = threadIdx.x;
-    const int kvh = blockIdx.y;
+    const int at = a.streams_first ? (int)blockIdx.z : (int)blockIdx.x;  // in the list of chunks
+    const int kvh = a.streams_first ? (int)blockIdx.x : (int)blockIdx.y;
+    const int layer = a.streams_first ? (int)blockIdx.y : (int)blockIdx.z;
     // the chunk's sequence: lane i compares the end of sequence i's chunks
     int s = 0;
     if (a.seqs > 1) {
-        const bool past = lane < a.seqs - 1 && a.first[lane + 1] <= (int)blockIdx.x;
+        const bool past = lane < a.seqs - 1 && a.first[lane + 1] <= at;
         s = __builtin_amdgcn_readfirstlane(__builtin_popcountll(__builtin_amdgcn_ballot_w64(past)));
     }
-    const int chunk_id = (int)blockIdx.x - a.first[s];
-    const int sl = s * a.layers + (int)blockIdx.z;
+    const int chunk_id = at - a.first[s];
+    const int sl = s * a.layers + layer;
     const int pos = a.positions[s];
     const int n_chunks = a.first[s + 1] - a.first[s];
     // (n_chunks = ceil(tiles / t) for some t, so no chunk is empty)
@@ -703,18 +706,36 @@ DecodeGeometry decode_geometry(const size_t *positions, size_t position, size_t 
     if (tiles < min_tiles) {
         tiles = min_tiles;
     }
-    // A batch: the longest sequence gets at least kBatchChunks chunks (of 8
-    // tiles or more, within the chunk bound, so the workspace stays as it
-    // is).  With one to three chunks per sequence their lengths differ by
-    // several times and the long ones run on alone: 7B, 8 ragged sequences of
-    // 1.5K-16K, 28 layers 707 us with 3 chunks of the longest, 655 with 4, 609
-    // with 6, 616 with 8; 3B, 4 ragged of 73-31K 464 and 440 us; a single
-    // sequence's chunks are equal, and there finer ones cost 2-8 %.
+    // A batch whose lengths differ: with one to three chunks per sequence the
+    // chunk lengths differ by several times and the long ones run on alone, so
+    // the longest sequence is cut into kBatchChunks chunks (of about 8 tiles or
+    // more, and within the chunk bound, so the workspace stays as it is): 7B, 8
+    // ragged sequences of 1.5K-16K, 28 layers 703 us with 2 chunks of the
+    // longest, 642 with 4, 598 with 6, 605 with 8.  Where the chunks' mean length
+    // is near the longest's there is little to even out and the finer cut only
+    // adds partials, 6 % of the cache bytes at 8 tiles and 8 heads per KV head
+    // (sequences of one length, 8 chunks against the cut above: 7B, 16 of 2048
+    // 374 against 306 us, 16 of 4096 668 against 590; 3B, 64 of 1024 502 against
+    // 422).  So the mean has to be under 0.7 of the longest where the finer chunks
+    // have 8 tiles or fewer, rising to 0.95 at 16 (7B, 8 of 11K-16K, mean 0.84:
+    // 1095 us with the cut above, 1018 with 8 chunks; 16 of 1.4K-2K, the same
+    // mean: 277 and 315).
+    bool refined = false;
     if (seqs > 1) {
         const size_t n = std::min(std::min(std::min(kBatchChunks, refine_chunks), (max_tiles + 7) / 8),
                                   decode_chunks_bound(max_n - 1, layers, kv_heads));
-        if (n > 0) {
-            tiles = std::min(tiles, (max_tiles + n - 1) / n);
+        const size_t finer = n > 0 ? (max_tiles + n - 1) / n : tiles;
+        size_t batch_tiles = 0, batch_chunks = 0;  // of one (layer, KV head)
+        for (size_t s = 0; s < seqs; ++s) {
+            const size_t t = ((positions != nullptr ? positions[s] : position) + kTile) / kTile;
+            batch_tiles += t;
+            batch_chunks += (t + tiles - 1) / tiles;
+        }
+        // in 256ths of the longest chunk: 0.45 + finer / 32 within 0.7 .. 0.95
+        const size_t even = std::min<size_t>(243, std::max<size_t>(179, 115 + 8 * finer));
+        if (finer < tiles && 256 * batch_tiles < even * batch_chunks * tiles) {
+            tiles = finer;
+            refined = true;
         }
     }
     size_t chunk = tiles * kTile;
@@ -730,6 +751,14 @@ DecodeGeometry decode_geometry(const size_t *positions, size_t position, size_t 
     }
     g.chunk = (int)chunk;
     g.max_chunks = (int)((max_n + chunk - 1) / chunk);
+    // Workgroups go to the XCDs round-robin.  With the chunk index fastest, the
+    // few long chunks of a batch (often a multiple of 8 of them) tie each
+    // sequence to one or two XCDs, so there the (KV head, layer) streams come
+    // first: 7B, 28 layers, 16 sequences of 2048 327 -> 306 us, 16 of 1K-2K 276 ->
+    // 250.  A refined batch's chunks are even over the XCDs in either order
+    // (7B, 8 of 1.5K-16K 602 us, 620 with the streams first), and chunks under
+    // 256 positions are faster chunk first (0.5B, 8 of 255 14.0 against 15.1).
+    g.streams_first = seqs > 1 && !refined && g.max_chunks <= 4 && g.chunk >= 8 * kTile;
     return g;
 }
 
@@ -742,7 +771,8 @@ size_t decode_workspace_bytes(const DecodeGeometry &g, size_t seqs, size_t layer
 size_t decode_chunks_bound(size_t max_position, size_t layers, size_t kv_heads) {
     // decode_geometry gives the longest stream n_longest = ceil(M / t0) chunks,
     // M = its 32-position tiles, t0 = max(2, ceil(T / target)) and T >= layers *
-    // kv_heads * M the total tiles; the later steps only lengthen the chunk.  So
+    // kv_heads * M the total tiles; the later steps only lengthen the chunk, but for
+    // a batch's finer cut, which takes no more chunks than this bound.  So
     // n_longest <= ceil(M / 2) and n_longest <= ceil(target / (layers * kv_heads)),
     // both non-decreasing in M.  One-tile chunks give n_longest = M where
     // layers * kv_heads * M <= T <= 3/4 of the CUs: at most
@@ -818,7 +848,7 @@ extern "C" size_t te_hip_attention_decode_workspace_bytes(const size_t *position
         const size_t p = positions != nullptr ? positions[s] : position;
         max_position = p > max_position ? p : max_position;
     }
-    te_hip::DecodeGeometry g;
+    te_hip::DecodeGeometry g = {};
     g.chunk = 0;
     g.max_chunks = (int)te_hip::decode_chunks_bound(max_position, layers, kv_heads);
     return te_hip::decode_workspace_bytes(g, seqs, layers, heads, head_dim);
@@ -888,7 +918,10 @@ te_status launch_splitk(const DecodeArgs &fused, bool is_fused, const float *que
         a.positions[s] = (int)(positions != nullptr ? positions[s] : position);
         a.first[s + 1] = a.first[s] + (int)chunks_of((size_t)a.positions[s], geo);
     }
-    const dim3 grid((unsigned)a.first[seqs], (unsigned)kv_heads, (unsigned)layers);
+    const unsigned chunks = (unsigned)a.first[seqs];
+    a.streams_first = geo.streams_first ? 1 : 0;
+    const dim3 grid = a.streams_first ? dim3((unsigned)kv_heads, (unsigned)layers, chunks)
+                                      : dim3(chunks, (unsigned)kv_heads, (unsigned)layers);
     hipStream_t strm = te_hip::as_stream(stream);
     if (head_dim == 128) {
         if (is_fused) {
@@ -1109,7 +1142,7 @@ extern "C" te_status te_hip_attention_decode_step_noalloc_f16(
     // The partials this exact call writes (not the position-monotone bound
     // the workspace query reports) must fit the array; a batch is cut no finer
     // than that.
-    const size_t per_chunk = te_hip::decode_workspace_bytes({0, 1}, seqs, layers, heads, head_dim);
+    const size_t per_chunk = te_hip::decode_workspace_bytes({0, 1, false}, seqs, layers, heads, head_dim);
     const size_t refine = (size_t)TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES / per_chunk;
     const te_hip::DecodeGeometry geo = te_hip::decode_geometry(positions, position, seqs, layers, kv_heads, refine);
     const size_t need = te_hip::decode_workspace_bytes(geo, seqs, layers, heads, head_dim);

@@ -78,8 +78,9 @@ inline te_status launch_status() {
 // Decode split-K geometry, shared by the split-K and combine launches and the
 // workspace-size query so all three agree.
 struct DecodeGeometry {
-    int chunk;       // most cache positions per workgroup (multiple of 32)
-    int max_chunks;  // chunks of the longest sequence
+    int chunk;           // most cache positions per workgroup (multiple of 32)
+    int max_chunks;      // chunks of the longest sequence
+    bool streams_first;  // order of the split-K workgroups: (KV head, layer) streams first, not chunks
 };
 
 // Compute units of the current device (256 when the query fails).
