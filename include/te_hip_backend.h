@@ -202,11 +202,15 @@ TE_API te_status te_hip_attention_decode_step_splitk_f16(
  * te_hip_attention_decode_step_f16 without the workspace: the split-K partials
  * go to a device array inside the library, TE_HIP_DECODE_NOALLOC_SCRATCH_BYTES
  * (16 MiB) per GPU, held from first use until the process ends.  The call
- * allocates nothing.  A call whose partials
- * (seqs*layers*heads*chunks*(head_dim+2)*4 bytes, chunks as reported by
- * te_hip_attention_decode_chunking) exceed the array takes the longer chunks
- * that fit it; one that fits with none returns TE_STATUS_UNSUPPORTED before
- * any work is queued.  Every call on one GPU
+ * allocates nothing.  The partials take seqs*layers*heads*chunks*(head_dim+2)*4
+ * bytes, chunks as reported by te_hip_attention_decode_chunking.  A batch that
+ * is cut finer than its size needs (to even out sequences of different
+ * lengths) and whose partials exceed the array so is cut less finely, down to
+ * the cut its size needs; its result then agrees with the workspace form's to
+ * fp32 rounding instead of bit for bit.  A call whose partials exceed the array
+ * even so, and any of a single sequence or of even lengths whose partials do,
+ * returns TE_STATUS_UNSUPPORTED before any work is queued: the chunks are not
+ * made longer than the size asks for.  Every call on one GPU
  * shares the array: calls that overlap in time on one GPU (different streams,
  * different threads) race and must be ordered by the caller.
  */

@@ -1,7 +1,8 @@
 """The cut of a decode batch into split-K chunks, on the host: a batch whose
 sequences are about as long as each other keeps the cut its size gives, a
-ragged one is cut finer, and neither needs more than the workspace query's
-bound (256 compute units, as without a device).
+ragged one is cut finer, neither needs more than the workspace query's bound,
+and the array-backed step refuses what its array cannot hold before any work
+(256 compute units, as without a device).
 """
 import ctypes
 import random
@@ -51,3 +52,17 @@ def test_no_batch_needs_more_than_its_workspace():
         arr = (ctypes.c_size_t * seqs)(*positions)
         held = lib.te_hip_attention_decode_workspace_bytes(arr, 0, seqs, layers, heads, kv, d)
         assert held >= seqs * layers * heads * _chunking(positions, layers, kv)[1] * (d + 2) * 4, positions
+
+
+def test_array_backed_step_refuses_a_cut_beyond_its_array():
+    """One long sequence among short ones: the chunks its size needs (342 of 3
+    tiles, 21.7 MiB of partials) exceed the 16 MiB array, though longer ones
+    would fit it.  Refused on the host: no pointer is used."""
+    layers, heads, kv, d, positions = 1, 16, 2, 128, [32767] + [1] * 7
+    chunks = _chunking(positions, layers, kv)[1]
+    assert chunks == 342 and len(positions) * layers * heads * chunks * (d + 2) * 4 > 16 << 20
+    arr = (ctypes.c_size_t * len(positions))(*positions)
+    p = ctypes.c_void_p(4096)
+    st = R.load_library().te_hip_attention_decode_step_noalloc_f16(
+        p, p, p, None, None, None, p, p, p, p, arr, 0, len(positions), layers, 32768, heads, kv, d, p, None)
+    assert st == R.TE_STATUS_UNSUPPORTED
