@@ -429,7 +429,7 @@ TE_API te_status te_hip_sample_top_k_f32(const float *logits, size_t vocab, uint
  * 2 SwiGLU (x is gate, x2 is up, as te_swiglu_f32).  W is a GGUF Q4_0 (2) or
  * Q8_0 (8) tensor [n][k] in device memory at a 2-byte aligned address,
  * k % 32 == 0.  Each activation enters as the sum of two bf16 values (error <=
- * 2^-18 of it), each weight code exactly; products are bf16 MFMA sums in fp32,
+ * 2^-17 of it from 2^-104 on, an absolute 2^-121 below), each weight code exactly; products are bf16 MFMA sums in fp32,
  * scaled and accumulated per 32-value block in fp32.  `act` is device
  * scratch of te_hip_gemm_act_bytes(rows, k) bytes.  `partials` (may be NULL)
  * is device scratch of partial_bytes bytes: with it, an output grid too small

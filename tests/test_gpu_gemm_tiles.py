@@ -4,9 +4,8 @@ block, odd and partial chunks of blocks, K splits with a short last part, and
 weights at 2- and 4-byte aligned addresses.
 
 Bound per output, against the fp64 product with the dequantized weights: each
-activation is the sum of two bf16 values within 2^-18 of it (twice that is
-allowed, for the second part's own rounding), the block sums and their
-accumulation are fp32 (a term is rounded at most 4 times per MFMA of 16 terms
+activation is the sum of two bf16 values within 2^-17 of it, the block sums and
+their accumulation are fp32 (a term is rounded at most 4 times per MFMA of 16 terms
 and once per block and split): (2^-17 + (k / 16 + 40) 2^-24) sum |w x|.
 """
 import numpy as np

@@ -7,10 +7,10 @@
 // Products (gemm_bf16_kernel): one 32-value block of a row against one GGUF
 // block of a weight row is two K = 16 steps of v_mfma_f32_32x32x16_bf16 for
 // each of two operand parts.  An activation x enters as hi + lo bf16 (hi =
-// RNE(x), lo = RNE(x - hi): |x - hi - lo| <= 2^-18 |x|, with the exponent
-// range of fp32), a weight code (Q4_0's n - 8, Q8_0's byte) as one bf16,
-// exactly.  The block's fp32 sum is scaled by the weight block's scale d and
-// accumulated in fp32, one FMA per product of the block.
+// RNE(x), lo = RNE(x - hi), 8 significant bits each: |x - hi - lo| <= 2^-17
+// |x|, with the exponent range of fp32), a weight code (Q4_0's n - 8, Q8_0's
+// byte) as one bf16, exactly.  The block's fp32 sum is scaled by the weight
+// block's scale d and accumulated in fp32, one FMA per product of the block.
 //
 // Why two bf16 parts and not integer digits: a block-scaled integer digit
 // form (two int8 MFMAs at twice the rate) needs a shift, a conversion and the
@@ -20,7 +20,8 @@
 //
 // Range: activations are stored times 2^-13 (kActScale) and the weight scales
 // times 2^13, so that a block's sum (32 products with codes up to 128) of
-// values near FLT_MAX stays finite, as the row's true sum does.
+// values near FLT_MAX stays finite, as the row's true sum does.  At the other
+// end lo is a subnormal bf16 for |x| < 2^-104: an absolute error of 2^-121 there.
 //
 // Layout of the activation operand (act_off): units of one 32-row tile and one
 // 32-value block, [M/32][K/32], 4 KiB each: [hi, lo][K step 0, 1][K half
