@@ -1516,6 +1516,12 @@ te_status launch_prefill(PrefillArgs a, size_t seqs, size_t layers, size_t token
 // 107 (3p); 7B 700 after 5000 87 (1u), 90 (3u); 1.5B 300 after 9000 128 (1u),
 // 45 (6u); 3B 64 after 2000 37 (1u), 23 (4u).  The smallest S with the least
 // time wins.  TE_HIP_PREFILL_SPLITS (1..32) overrides the choice.
+//   One split over few keys is the rows kernel for fp32 queries (prefill_rows),
+// whose time does not go in steps of 128 keys but grows by 0.4 us over the last
+// step before kRowsMaxKeysQ32, whatever the rows.  Fused step, one split (rows
+// kernel) / 4 splits, us, at 416 and 512 keys: 7B 24 rows 16.5 / 15.4 and 17.2 /
+// 15.5, 40 rows 16.6 / 16.5 and 17.3 / 16.6, 64 rows 16.6 / 17.8 and 17.4 / 18.2;
+// 3B 4 rows 16.1 / 14.1 and 16.9 / 14.1, 48 rows 16.5 / 16.1 and 17.2 / 16.2.
 int prefill_splits(size_t seqs, size_t layers, size_t tokens, size_t base_position, size_t heads,
                    size_t head_dim, size_t max_splits = kMaxPrefillSplits) {
     const size_t n_qtiles = (tokens + BM - 1) / BM;
@@ -1532,6 +1538,8 @@ int prefill_splits(size_t seqs, size_t layers, size_t tokens, size_t base_positi
         }
     }
     const double bytes = (double)(seqs * layers * tokens * heads * (head_dim + 2) * sizeof(float));
+    const size_t keys = base_position + tokens;
+    const double rows_us = keys <= kRowsMaxKeysQ32 ? 0.4 * (double)((keys - 1) % 128 + 1) / 128.0 : 0.0;
     auto launch_us = [&](size_t sp) {
         const bool paired = prefill_paired(seqs, layers, tokens, heads, (int)sp);
         const size_t units = (paired ? (n_qtiles + 1) / 2 : n_qtiles) * heads * seqs * layers * sp;
@@ -1544,7 +1552,7 @@ int prefill_splits(size_t seqs, size_t layers, size_t tokens, size_t base_positi
     };
     const size_t max_steps = tile_steps(n_qtiles - 1) + (n_qtiles > 1 ? tile_steps(0) : 0);
     size_t best = 1;
-    double best_us = launch_us(1);
+    double best_us = launch_us(1) + rows_us;
     for (size_t sp = 2; sp <= std::min<size_t>(kMaxPrefillSplits, max_splits) && sp <= max_steps; ++sp) {
         const double us = launch_us(sp);
         if (us < best_us && sp * seqs * layers <= 65535) {
