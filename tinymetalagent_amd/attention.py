@@ -50,9 +50,11 @@ _F32, _F16 = torch.float32, torch.float16
 
 
 def _step_dtypes(q, k, v, key_cache, value_cache) -> None:
-    """The dtypes of a fused step's tensors (the common case in one test)."""
-    if not (q.dtype is _F32 and k.dtype is _F32 and v.dtype is _F32 and key_cache.dtype is _F16
-            and value_cache.dtype is _F16):
+    """The dtypes of a fused step's tensors (the common case in one test; a
+    missing one is refused by the library)."""
+    if (k is None or v is None or value_cache is None
+            or not (q.dtype is _F32 and k.dtype is _F32 and v.dtype is _F32 and key_cache.dtype is _F16
+                    and value_cache.dtype is _F16)):
         for t, dt, n in ((q, _F32, "query"), (k, _F32, "k_new"), (v, _F32, "v_new"), (key_cache, _F16, "key_cache"),
                          (value_cache, _F16, "value_cache")):
             _dtype(t, dt, n)
