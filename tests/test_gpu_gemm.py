@@ -2,10 +2,10 @@
 row of the product against the fp64 product of the oracle's pre-op output
 and dequantized weights.
 
-Bound per output: 2^-14 sum_blocks max|x_block| sum_block |w| (the
-activations' 15-bit block rounding) + (blocks + 2) 2^-24 sum |w x| (fp32
-accumulation per block) + 2^-21 sum |w x| (the pre-op's last bits: RMSNorm and
-SwiGLU within 2 ulps of the oracle's).
+Bound per output, times sum |w x|: 2^-17 (an activation as two bf16 values; an
+absolute 2^-121 below 2^-104) + (k / 16 + blocks + 2) 2^-24 (fp32 sums: at most
+four roundings of a term per MFMA of 16, one per block) + 2^-21 (the pre-op's
+last bits: RMSNorm and SwiGLU within 2 ulps of the oracle's).
 """
 import ctypes
 
@@ -48,10 +48,8 @@ def _run(oracle_mod, ggml_type, rows, n, k, pre=0, resid=False, seed=3, scale=1.
     exact = xp.astype(np.float64) @ wf.T
     if resid:
         exact += r
-    ax = np.abs(xp.astype(np.float64))
-    bmax = np.repeat(ax.reshape(rows, k // 32, 32).max(2), 32, axis=1)
-    awx = ax @ np.abs(wf).T
-    bound = 2.0 ** -14 * (bmax @ np.abs(wf).T) + ((k // 32 + 2) * 2.0 ** -24 + 2.0 ** -21) * awx + 1e-30
+    awx = np.abs(xp.astype(np.float64)) @ np.abs(wf).T
+    bound = (2.0 ** -17 + (k / 16 + k // 32 + 2) * 2.0 ** -24 + 2.0 ** -21) * awx + 2.0 ** -121 * np.abs(wf).sum(1)
     if resid:
         bound += 2.0 ** -24 * (np.abs(r) + awx)
     dw, dx, dx2, dn, dr = _dev(w), _dev(x), _dev(x2), _dev(nw), _dev(r)
@@ -71,8 +69,7 @@ def _run(oracle_mod, ggml_type, rows, n, k, pre=0, resid=False, seed=3, scale=1.
 
 @pytest.mark.parametrize("ggml_type,rows,n,k", [
     (2, 1, 64, 64), (2, 7, 100, 96), (8, 64, 64, 2048), (2, 130, 257, 256), (8, 65, 33, 512), (2, 256, 512, 2048),
-    # Q8_0 stages a weight chunk of 8 blocks in two halves: one partial chunk
-    # (no second half staged ahead), and a full chunk then a partial one
+    # a weight chunk is 4 blocks: one partial chunk, and full ones then a partial one
     (8, 7, 100, 96), (8, 130, 257, 288)])
 def test_gemm_vs_fp64(oracle_mod, ggml_type, rows, n, k):
     _run(oracle_mod, ggml_type, rows, n, k)
@@ -99,8 +96,8 @@ def test_gemm_input_ranges(oracle_mod):
     lib = R.load_library()
     for scale in (1e-30, 1e-3, 1e30):
         _run(oracle_mod, 2, 40, 64, 256, scale=scale)
-    # finite blocks whose largest magnitude is in (3e38, FLT_MAX] take the finite
-    # scale 2^114 (small weights keep every block sum inside fp32)
+    # values up to FLT_MAX are stored times 2^-13, so their block sums stay finite
+    # (small weights keep every output inside fp32)
     got = _run(oracle_mod, 2, 2, 40, 64, scale=3.3e38, clip=1.0, w_scale=1e-3)
     assert np.isfinite(got).all()
 
