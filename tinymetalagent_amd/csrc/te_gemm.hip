@@ -964,7 +964,14 @@ te_status launch_gemm_glu_q(uint32_t ggml_type, const void *gate_w, const void *
     sg.n_off[1] = (int)n;
     const bool w4 = rows_w4(gate_w, row_bytes) && rows_w4(up_w, row_bytes);
     GemmPlan plan = gemm_plan(rows, n, n_tiles, k / 32, 1);
-    // one projection's groups: the sums are those of the two GEMMs, bit for bit
+    // The groups that one projection's tiles take in one K split: where the two
+    // GEMMs run unsplit too, the sums are theirs bit for bit (the layer flow's
+    // partials let them split K at few rows, 3B and 1.5B at 8-64: not there).
+    // Where the pair's own tiles exceed the CUs and one projection's do not, its
+    // own plan would take one-group workgroups, two per CU; the override against
+    // that, two layers, us: 7B 8 / 64 / 128 rows Q4_0 291 : 295, 336 : 342, 461 :
+    // 436, Q8_0 383 : 410, 417 : 445, 522 : 541; 3B Q4_0 129 / 256 rows 284 : 269,
+    // 314 : 301; 1.5B 129 / 256 207 : 197, 257 : 243; 0.5B 512 rows 227 : 213.
     plan.groups = gemm_plan(rows, n, (n + kBN - 1) / kBN, k / 32, 1).groups;
     *launched = true;
     return launch_tiles(ggml_type, true, w4, sg, row_bytes, act, rows, k, plan, n_tiles, nullptr, act_out, stream);
