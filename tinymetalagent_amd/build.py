@@ -47,15 +47,13 @@ HIP_FLAGS = [
     "-Wall",
     "-Wno-unused-command-line-argument",
 ]
-# Per-source additions.  te_gemm.hip: MFMA results in VGPRs rather than
-# accumulation registers (its blocks' sums are scaled by VALU code).
-# te_vecops.hip and te_gemm.hip: the iterative-ilp scheduling strategy (the
-# 3B decode token Q4_0 1,431 -> 1,404 us, Q8_0 1,646 -> 1,627 us, same box,
-# alternating builds; the prompt GEMM within 1 % of the default strategy).  The
-# prefill, decode and append sources measured no better with it or the other
-# strategies.
+# Per-source additions.  te_vecops.hip and te_gemm.hip: the iterative-ilp
+# scheduling strategy (the 3B decode token Q4_0 1,431 -> 1,404 us, Q8_0 1,646 ->
+# 1,627 us, same box, alternating builds; the prompt GEMM within 1 % of the
+# default strategy).  The prefill, decode and append sources measured no better
+# with it or the other strategies.
 HIP_SOURCE_FLAGS = {
-    "te_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+    "te_gemm.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
     "te_vecops.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
 }
 
