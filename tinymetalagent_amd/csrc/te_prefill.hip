@@ -1432,10 +1432,10 @@ bool prefill_paired(size_t seqs, size_t layers, size_t tokens, size_t heads, int
 // for fp16 queries the choice stops at 256.  With fp32 queries (the fused
 // step: bias and RoPE on load) the tile kernel's query preparation costs
 // more than the rows kernel's (which loads a group's queries once, into
-// LDS), so the fused step takes the rows kernel up to kRowsMaxKeysQ32:
-// its attention at 3B L = 512 15.3 against 23.5 us, the 3B Q4_0 512-token
-// prompt 12.81 -> 12.43-12.67 ms.  TE_HIP_PREFILL_ROWS=1 takes it for every
-// launch with one split, =0 never.
+// LDS), so the fused step takes the rows kernel up to kRowsMaxKeysQ32: its
+// attention at 3B L = 512 14.6 against 16.2 us, in the prompt flow, with the
+// output projection's operand in place of fp32 rows, 17.8 against 20.6.
+// TE_HIP_PREFILL_ROWS=1 takes it for every launch with one split, =0 never.
 constexpr size_t kRowsMaxKeys = 256;
 constexpr size_t kRowsMaxKeysQ32 = 512;
 
