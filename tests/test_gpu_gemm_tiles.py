@@ -51,3 +51,23 @@ def test_gemm_tile_edges(oracle_mod, ggml_type, rows, n, k, split, shift):
     err = np.abs(got[:rows * n].reshape(rows, n) - exact)
     print(f"type {ggml_type} {rows}x{n}x{k}: max err / bound {float((err / bound).max()):.3f}")
     assert np.all(err <= bound)
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 64), (31, 96, 64), (65, 129, 96), (200, 300, 512)])
+def test_residual_in_place(rows, n, k):
+    """The residual added in the GEMM's own stores (one K split) with out ==
+    resid, as the layer flow passes it: the bits of separate buffers."""
+    lib = R.load_library()
+    w = torch.from_numpy(S.ggml_tensor(12, f"rw{n}{k}", 8, n, k, scale=0.05)).cuda()
+    x, r = (torch.from_numpy(S.normal(12, name, shape)).cuda() for name, shape in (("rx", (rows, k)), ("rr", (rows, n))))
+    act = torch.empty(lib.te_hip_gemm_act_bytes(rows, k), dtype=torch.uint8, device="cuda")
+
+    def gemm(out, resid):
+        R.check(lib.te_hip_gemm_q_f32(w.data_ptr(), 8, x.data_ptr(), None, None, 1e-6, 0, rows, n, k, out.data_ptr(),
+                                      resid, act.data_ptr(), None, 0, None))
+        return out
+
+    want = gemm(torch.empty(rows, n, device="cuda"), r.data_ptr())
+    plain = gemm(torch.empty(rows, n, device="cuda"), None)
+    here = r.clone()
+    assert torch.equal(gemm(here, here.data_ptr()), want) and torch.equal(want, r + plain)
