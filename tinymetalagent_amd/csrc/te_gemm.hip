@@ -219,7 +219,7 @@ typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // MFMAs alone on random operands runs at 1.75 PFLOP/s (the clock falls to 1.8
 // GHz); with the FMAs and LDS reads of a step 1.45, with the conversion 1.3.
 // Gate and up of 512 rows at 3B (2 x 11008 x 2048 Q4_0, 92 GFLOP of MFMA) take
-// 105 us, Q8_0 113 us, against 146 and 171 us with the block-scaled int8 digits
+// 98-104 us, Q8_0 108-117 us, against 146 and 171 us with the block-scaled int8 digits
 // this replaced; converting the weights costs 15 us of it, their loads 5.
 //
 // GLU: sg.w[0] / sg.w[1] are the gate / up matrices (n rows each); the tile's
@@ -777,8 +777,9 @@ te_status launch_split_act(int pre, const float *x, const float *x2, const float
 //   One round: two groups per workgroup.  A pair of chunks takes 3.4 us at 128
 //   rows on 64 CUs and 4.9 on all 256 (the clock falls), 2.5 and 3.0 at 64.
 //   More: two one-group workgroups per CU, which fill each other's waits (512
-//   x 22016 x 2048 Q4_0 109.7 us against 120.2 in two-group workgroups, Q8_0
-//   118.3 against 129.7); a round's pair takes 4.2 and 2.8 us.
+//   x 22016 x 2048 Q4_0 107-111 us against 110 in two-group workgroups, Q8_0
+//   111-113 against 116; 512 x 37888 x 3584 274-276 against 276-277, 296-299
+//   against 302-304); a round's pair takes 4.2 and 2.8 us.
 // The partial sums are written and read back at 2.7 TB/s.
 struct GemmPlan {
     int wm, groups;
@@ -997,9 +998,9 @@ te_status launch_gemm_glu_q(uint32_t ggml_type, const void *gate_w, const void *
     // partials let them split K at few rows, 3B and 1.5B at 8-64: not there).
     // Where the pair's own tiles exceed the CUs and one projection's do not, its
     // own plan would take one-group workgroups, two per CU; the override against
-    // that, two layers, us: 7B 8 / 64 / 128 rows Q4_0 291 : 295, 336 : 342, 461 :
-    // 436, Q8_0 383 : 410, 417 : 445, 522 : 541; 3B Q4_0 129 / 256 rows 284 : 269,
-    // 314 : 301; 1.5B 129 / 256 207 : 197, 257 : 243; 0.5B 512 rows 227 : 213.
+    // that, two layers, us: 7B 8 / 64 / 128 rows Q4_0 284 : 290, 325 : 333, 448 :
+    // 442, Q8_0 374 : 405, 405 : 438, 519 : 543; 3B Q4_0 129 / 256 rows 270 : 263,
+    // 311 : 301; 1.5B 129 / 256 192 : 187, 250 : 235; 0.5B 512 rows 207 : 196.
     plan.groups = gemm_plan(rows, n, (n + kBN - 1) / kBN, k / 32, 1).groups;
     *launched = true;
     return launch_tiles(ggml_type, true, w4, sg, row_bytes, act, rows, k, plan, n_tiles, nullptr, act_out, stream);
